@@ -944,7 +944,8 @@ int dfl_a2t_bwd(const dfl_a2t_params* p, void* workspace, size_t workspace_bytes
 size_t dfl_dense_sinkhorn_workspace_size(int B, int H, int N, int K) {
   if (B <= 0 || H <= 0 || N <= 0 || K < 0) return 0;
   const size_t bhn = (size_t)B * H * N;
-  return ((size_t)2 * (K + 1) * 4 + 255) / 256 * 256 + (2 * bhn * 4 + 255) / 256 * 256;
+  const size_t slots = (size_t)(K < dfl::DENSE_SEG ? K : dfl::DENSE_SEG) + 1;
+  return ((size_t)2 * (K + 1) * 4 + 255) / 256 * 256 + 2 * ((slots * bhn * 4 + 255) / 256 * 256);
 }
 
 int dfl_dense_sinkhorn_fwd(const dfl_dense_sinkhorn_params* p, void* workspace, size_t workspace_bytes,
@@ -1021,7 +1022,8 @@ int dfl_dense_sinkhorn_bwd(const dfl_dense_sinkhorn_bwd_params* p, void* workspa
   unsigned char* ws = static_cast<unsigned char*>(workspace);
   float* vecs = reinterpret_cast<float*>(ws + ((size_t)2 * (p->K_max + 1) * 4 + 255) / 256 * 256);
   a.gv = vecs;
-  a.avec = vecs + bhn;
+  const size_t slots = (size_t)(p->K_max < dfl::DENSE_SEG ? p->K_max : dfl::DENSE_SEG) + 1;
+  a.avec = vecs + (slots * bhn * 4 + 255) / 256 * 64;
   hipStream_t s = (hipStream_t)stream;
   hipError_t e;
   if (p->K == 0) {  // outputs are the (masked) initial potentials: dC, d log mu, d log nu vanish

@@ -26,6 +26,9 @@ struct DenseSinkArgs {
   float* log_v;
 };
 
+// iterations whose vectors the solver's backward keeps before it forms their cost gradient
+constexpr int DENSE_SEG = 16;
+
 // sinkhorn_solve backward through the K executed iterations.
 struct DenseSinkBwdArgs {
   const float* C;
@@ -44,8 +47,9 @@ struct DenseSinkBwdArgs {
   float* dlog_nu;
   float* dlog_u_init;   // or null
   float* dlog_v_init;   // or null
-  float* gv;            // workspace (B,H,N): g_v of the current iteration
-  float* avec;          // workspace (B,H,N): -kappa g_u of the current iteration
+  // workspace rings of min(K, DENSE_SEG) + 1 slots of (B,H,N); iteration k uses slot (K - k) % (DENSE_SEG + 1)
+  float* gv;            // g_v(k)
+  float* avec;          // -kappa g_u(k)
 };
 
 // compute_transport_output forward / backward.  V, G, o_avg, goa (B,H,N,d) with d <= 64.

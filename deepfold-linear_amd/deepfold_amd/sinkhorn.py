@@ -46,6 +46,7 @@ class _DenseSinkhorn(torch.autograd.Function):
         _lib.check(rc, "dfl_dense_sinkhorn_fwd")
         ctx.save_for_backward(Cf, ep, m, history)
         ctx.meta = (B, H, N, int(K), done.value, float(lam), log_u_init is not None, log_v_init is not None)
+        ctx.set_materialize_grads(False)  # a missing gradient is a NULL of the C ABI, not a zero tensor
         return log_u, log_v
 
     @staticmethod
@@ -127,6 +128,7 @@ class _DenseTransport(torch.autograd.Function):
         _lib.check(rc, "dfl_dense_transport_fwd")
         ctx.save_for_backward(Vf, Gf, lu, lv, Cf, ep, x, m, T_norm, o_avg)
         ctx.meta = (B, H, N, d)
+        ctx.set_materialize_grads(False)  # above all for T_norm: no (B,H,N,N) zeros to fill and read
         return o, T_norm, xc
 
     @staticmethod

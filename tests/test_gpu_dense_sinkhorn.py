@@ -201,3 +201,32 @@ def test_solve_then_transport_masked_pipeline():
     _cmp(out, ("C", "mu", "nu", "V", "G", "x"))
     o = out["gpu"][1]["o"].detach().cpu()
     assert torch.all(o[1, 40:] == 0)
+
+
+@pytest.mark.parametrize("B,H,N,d,K,lengths", [
+    (1, 1, 1040, 20, 3, None),       # rows longer than the 1024 columns held at once; d not a whole tile
+    (1, 1, 1027, 64, 2, None),       # the same with rows that are not 16-byte aligned
+    (1, 2, 36, 16, 35, None),        # three segments of the 16 iterations whose cost gradient is formed at once
+    (2, 2, 97, 32, 17, [97, 50]),    # one iteration past a segment; ragged edges of every tile
+    (1, 1, 1, 3, 2, None),           # a single token
+])
+def test_pipeline_tile_edges(B, H, N, d, K, lengths):
+    """Solver into transport where its tiles, chunks and segments end (fp32: the bar of this file)."""
+    print(f"case B{B} H{H} N{N} d{d} K{K}", flush=True)
+    C, lmu, lnu, eps, g = _case(B, H, N, seed=N + d)
+    mask = None if lengths is None else _mask(B, N, lengths)
+    V, G = torch.randn(B, H, N, d, generator=g), torch.randn(B, H, N, d, generator=g)
+    x = torch.randn(B, N, 3, generator=g)
+    wo, wx = torch.randn(B, N, H * d, generator=g), torch.randn(B, H, N, 3, generator=g)
+    wT = torch.randn(B, H, N, N, generator=g)
+
+    def fn(ls, tag):
+        cw = (lambda t: None if t is None else t.double()) if tag == "ref" else \
+            (lambda t: None if t is None else t.float().to(DEV))
+        lu, lv = _solve(tag)(ls["C"], ls["mu"], ls["nu"], cw(eps), K=K, mask=cw(mask))
+        o, Tn, xc = _transport(tag)(ls["V"], ls["G"], lu, lv, ls["C"], cw(eps), ls["x"], cw(mask))
+        return (o * cw(wo)).sum() + (xc * cw(wx)).sum() + (Tn * cw(wT)).sum(), {"o": o, "x_centroid": xc, "T": Tn}
+
+    # a single row's plan is 1 whatever the cost: its cost and marginal gradients vanish
+    names = ("V", "G", "x") if N == 1 else ("C", "mu", "nu", "V", "G", "x")
+    _cmp(_grads(fn, {"C": C, "mu": lmu, "nu": lnu, "V": V, "G": G, "x": x}), names)
