@@ -508,14 +508,12 @@ int run_fwd(dfl::SinkFwdArgs& a, bool bf16, int DP, int storage, const FwdScratc
   // geometry term, whose per-element cost it computes once instead of every sweep
   const bool has_bias = (a.bins && a.pos_w) || (a.x && a.w_dist);
   const size_t lds_reg = dfl::sinkhorn_fwd_reg_lds_bytes(a.N, DP, elem, G);
-  const bool reg_ok = !a.balanced && !a.hist && a.K_iter >= 1 && dfl::sinkhorn_fwd_reg_fits(a.N, G) &&
-                      lds_reg <= LDS_LIMIT;
+  const bool reg_ok = a.K_iter >= 1 && dfl::sinkhorn_fwd_reg_fits(a.N, G) && lds_reg <= LDS_LIMIT;
   const bool blk_mode =
       blk_ok && (storage == DFL_STORAGE_REGISTER || (storage == DFL_STORAGE_AUTO && has_bias && !reg_ok));
   const bool stream_mode =
       !blk_mode && (storage == DFL_STORAGE_STREAM || (storage == DFL_STORAGE_AUTO && lds_res > LDS_LIMIT));
-  // resident layout with the logits in registers: the UOT forward without history whose
-  // stripes and slots fit the register tiles
+  // resident layout with the plan in registers, where the stripes and slots fit the register tiles
   const bool reg_mode = !blk_mode && !stream_mode && storage == DFL_STORAGE_AUTO && reg_ok;
   const size_t lds = blk_mode ? lds_blk
                               : (stream_mode ? dfl::sinkhorn_fwd_lds_bytes(a.N, DP, elem, G, true)

@@ -6,6 +6,8 @@
 // resident rows are Q (plan rows i) and the streamed rows are K (plan columns
 // j); in a column sweep the roles swap.  NT = threads per workgroup.
 #pragma once
+#include <type_traits>
+
 #include "common.h"
 #include "sinkhorn_args.h"
 
@@ -58,6 +60,30 @@ struct Bias {
     if (b8) b += posw[b8[(size_t)i * Np + j]];
     if (xs) b += geo(xs[3 * i] - xs[3 * j], xs[3 * i + 1] - xs[3 * j + 1], xs[3 * i + 2] - xs[3 * j + 2]);
     return b;
+  }
+  // quads for one streamed tile, in two steps (bins, not the matrices): the bin word of
+  // resident index r at streamed indices s0..s0+3, and the biases from it.
+  template <bool COL> __device__ __forceinline__ uint32_t word(int r, int s0) const {
+    return b8 ? *reinterpret_cast<const uint32_t*>((COL ? b8t : b8) + (size_t)r * Np + s0) : 0u;
+  }
+  __device__ __forceinline__ f32x4 from_word(uint32_t w, int r, int s0) const {
+    f32x4 out = {0.f, 0.f, 0.f, 0.f};
+    if (b8) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) out[e] = posw[(w >> (8 * e)) & 0xffu];
+    }
+    if (xs) {
+      const float r0x = xs[3 * r], r1x = xs[3 * r + 1], r2x = xs[3 * r + 2];
+      const float* c = xs + 3 * s0;
+      const f32x4 p = *reinterpret_cast<const f32x4*>(c);
+      const f32x4 q = *reinterpret_cast<const f32x4*>(c + 4);
+      const f32x4 t = *reinterpret_cast<const f32x4*>(c + 8);
+      out[0] += geo(r0x - p[0], r1x - p[1], r2x - p[2]);
+      out[1] += geo(r0x - p[3], r1x - q[0], r2x - q[1]);
+      out[2] += geo(r0x - q[2], r1x - q[3], r2x - t[0]);
+      out[3] += geo(r0x - t[1], r1x - t[2], r2x - t[3]);
+    }
+    return out;
   }
   // The biases of resident index r against the four streamed indices s0[k]..s0[k]+3
   // of each of S streamed tiles (s0 % 4 == 0, s0 + 3 < Np).  COL: the streamed
@@ -684,66 +710,95 @@ template <> __device__ __forceinline__ f32x4 reg_pv<float>(const float (&p)[4], 
 // after the chunk's barrier (flow_chunk), the only barrier of a half-iteration
 // with at most 4 resident tiles (2 with a bias).
 
-// Polls the words of this wave's streamed tiles (entries i < n) until they carry
-// `tag`, writes dst[i] = word * log2 e (NEG_BIG for a masked entry), and its split
-// parts[i] = split3(dst[i]) if parts is given, and sets dmax, in every lane, to the
-// largest |change| over the wave's valid entries (+inf for a NaN).  Returns false,
-// uniformly over the wave, if a wait expired (then the error has been raised).
-template <int NW>
-__device__ __forceinline__ bool wave_gather(const uint64_t* buf, int n, int n_tiles, uint32_t tag, float* dst,
-                                            const unsigned char* valid, ErrRef err, float& dmax,
-                                            bf16x4* parts = nullptr) {
+// Polls the words of this wave's streamed tiles (entries i < n) until they carry `tag`,
+// hands each entry and its new value word * log2 e (NEG_BIG for a masked entry, and at least
+// NEG_BIG) to take(s, i, value, valid), s = 0, 1, ... the lane's entries in order, which returns
+// its |change|, and sets dmax, in every lane, to the largest of them over the wave.  MAXW: most
+// entries of a lane (a wave's words over 64), 0 for any number (s is then 0 or 1).  Returns false, uniformly over the wave, if a wait
+// expired (then the error has been raised).
+template <int NW, int MAXW, typename Take>
+__device__ __forceinline__ bool wave_poll(const uint64_t* buf, int n, int n_tiles, uint32_t tag,
+                                          const unsigned char* valid, ErrRef err, float& dmax, Take take) {
   const int lane = threadIdx.x & (WAVE - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int nwords = wave < n_tiles ? ((n_tiles - 1 - wave) / NW + 1) * 16 : 0;
   float dm = 0.f;
   bool ok = true;
-  for (int base = 0; base < nwords && ok; base += 2 * WAVE) {
-    int idx[2];
+  const auto batch = [&](auto wc, int base) __attribute__((always_inline)) {
+    constexpr int W = decltype(wc)::value;
+    int idx[W];
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
+    for (int k = 0; k < W; ++k) {
       const int e = base + k * WAVE + lane;
       const int i = (wave + NW * (e >> 4)) * 16 + (e & 15);
       idx[k] = (e < nwords && i < n) ? i : -1;
     }
-    ok = poll_words<2>(buf, idx, tag, err, [&](int k, uint64_t w) {
+    ok = poll_words<W>(buf, idx, tag, err, [&](int k, uint64_t w) {
       const int i = idx[k];
-      float nv = NEG_BIG;
-      if (valid[i]) {
-        nv = __uint_as_float((uint32_t)(w >> 32)) * LOG2E;
-        dm = fmaxf(dm, fabsf(nv - dst[i]));
-      }
-      dst[i] = nv;
-      if (parts) parts[i] = split3(nv);
+      const float nv = __uint_as_float((uint32_t)(w >> 32)) * LOG2E;
+      dm = fmaxf(dm, valid[i] ? take(k, i, nv < NEG_BIG ? NEG_BIG : nv, true) : take(k, i, NEG_BIG, false));
     });
     ok = wave_max_u32(ok ? 0u : 1u) == 0u;
+  };
+  static_assert(MAXW <= 2, "at most two words a lane at once");
+  if constexpr (MAXW == 0) {
+    for (int base = 0; base < nwords && ok; base += 2 * WAVE) batch(std::integral_constant<int, 2>{}, base);
+  } else {
+    if (nwords > 0) batch(std::integral_constant<int, MAXW>{}, 0);
   }
   dmax = __uint_as_float(wave_max_u32(dm == dm ? __float_as_uint(dm) : 0x7f800000u));
   return ok;
+}
+// wave_poll into dst[i]; dmax is the largest |change| of a valid entry.
+template <int NW>
+__device__ __forceinline__ bool wave_gather(const uint64_t* buf, int n, int n_tiles, uint32_t tag, float* dst,
+                                            const unsigned char* valid, ErrRef err, float& dmax) {
+  return wave_poll<NW, 0>(buf, n, n_tiles, tag, valid, err, dmax, [&](int, int i, float nv, bool ok) {
+    const float d = ok ? fabsf(nv - dst[i]) : 0.f;
+    dst[i] = nv;
+    return d;
+  });
+}
+// wave_poll into dst[i] and the multipliers w[i] = exp2(dst[i] - base) of scaling form (0 for a
+// masked entry), with the bases in registers: base[s] of entry 64 s + lane of the wave's words
+// (the wave's tiles in order, 16 entries each).  dmax is the largest |dst - base| of a valid entry.
+template <int NW, int NB>
+__device__ __forceinline__ bool wave_gather_scaled(const uint64_t* buf, int n, int n_tiles, uint32_t tag, float* dst,
+                                                   const float (&base)[NB], float* w, const unsigned char* valid,
+                                                   ErrRef err, float& dmax) {
+  return wave_poll<NW, NB>(buf, n, n_tiles, tag, valid, err, dmax, [&](int s, int i, float nv, bool ok) {
+    const float d = nv - base[s];
+    dst[i] = nv;
+    w[i] = ok ? fast_exp2(d) : 0.f;
+    return ok ? fabsf(d) : 0.f;
+  });
 }
 
 // Combine of the NW wave partials part[q * NW + w] of the nr * 16 rows q (threads
 // q < 16 nr): lse[q] = m + log2 sum_w exp2(p_w - m), m = max_w p_w, in wave order,
 // then publish(q, lse[q]).  A row's partials are adjacent: 16-byte reads.
+template <int NW> __device__ __forceinline__ float flow_lse(const float* part, int q) {
+  static_assert(NW % 4 == 0, "partials are read 4 at a time");
+  float p[NW];
+#pragma unroll
+  for (int w4 = 0; w4 < NW; w4 += 4) {
+    const f32x4 v = *reinterpret_cast<const f32x4*>(part + q * NW + w4);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) p[w4 + k] = v[k];
+  }
+  float m = p[0];
+#pragma unroll
+  for (int w_ = 1; w_ < NW; ++w_) m = fmaxf(m, p[w_]);
+  float ss = 0.f;
+#pragma unroll
+  for (int w_ = 0; w_ < NW; ++w_) ss += fast_exp2(p[w_] - m);
+  return m + fast_log2(ss);
+}
 template <int NW, typename Pub>
 __device__ __forceinline__ void flow_combine(const float* part, int nr, float* lse, Pub publish) {
-  static_assert(NW % 4 == 0, "partials are read 4 at a time");
   if ((int)threadIdx.x < nr * 16) {
     const int q = threadIdx.x;
-    float p[NW];
-#pragma unroll
-    for (int w4 = 0; w4 < NW; w4 += 4) {
-      const f32x4 v = *reinterpret_cast<const f32x4*>(part + q * NW + w4);
-#pragma unroll
-      for (int k = 0; k < 4; ++k) p[w4 + k] = v[k];
-    }
-    float m = p[0];
-#pragma unroll
-    for (int w_ = 1; w_ < NW; ++w_) m = fmaxf(m, p[w_]);
-    float ss = 0.f;
-#pragma unroll
-    for (int w_ = 0; w_ < NW; ++w_) ss += fast_exp2(p[w_] - m);
-    const float v = m + fast_log2(ss);
+    const float v = flow_lse<NW>(part, q);
     lse[q] = v;
     publish(q, v);
   }
@@ -897,23 +952,31 @@ __device__ __forceinline__ void flow_sweep(bool online, const T* res, const T* s
 }
 
 // ---------------------------------------------------------------------------
-// Register storage of the resident layout.  A wave keeps the logits of its (resident
-// tile r, streamed slot k) pairs in VGPRs, S[r KS + k] for r < nr, k < KS (streamed
-// tile st = wave + NW k; slots of tiles the wave does not have hold NEG_BIG), computed
-// once per launch.  A sweep adds the potentials with one rank-2 MFMA per pair
-// (streamed term in the A operand, -shift of the resident row in B) and sums exp2;
-// each row's partial p_w goes to part as in flow_chunk.  Online (the first sweep, or
-// a wave whose streamed potentials moved by more than the fixed-shift bound) takes
-// the row maxima of its pairs first and uses them as its shifts.
-//   colp : split parts of the streamed potentials (by absolute streamed index)
-//   rowp : split parts of -shift of the resident rows (local), for the fixed mode
-//   shift: the fixed shifts (local rows)
-// pmax (online only): the wave's row maxima, pmax[(r 16 + l) NW + wave], NEG_BIG
-// where the wave has no live entry.
+// Register storage of the resident layout.  A wave keeps the plan entries of its (resident
+// tile r, streamed slot k) pairs in VGPRs, X[r KS + k] for r < nr, k < KS (streamed tile
+// st = wave + NW k), in scaling form: E_ij = exp2(S_ij + base_j - sh_i) with base_j the
+// streamed potential and sh_i the wave's row maximum of S + base at the time they were
+// formed.  A sweep then is one multiply-add per element, sum_j E_ij w_j with w_j =
+// exp2(pot_j - base_j), where the logits with an exponential per element and sweep took a
+// rank-2 MFMA, four exponentials and four adds a pair: at the headline's 759-token
+// members 1.05-1.35 us a sweep before, about 0.35 us so.  E <= 1, so an entry that
+// underflows is below 2^-126 of its row's largest; while no potential has moved by more than
+// REG_MAX_DRIFT from its base, it stays below 2^-62 of it.  A wave that meets a larger move
+// leaves REG_REDO as its partials; the workgroup then forms its entries anew and repeats the
+// sweep, which nothing has been published of.  Once a row's LSE of the sweep that formed its
+// entries is known, every wave brings them to that common shift (reg_rescale), so the later
+// partials of the waves are plain sums.
+constexpr float REG_MAX_DRIFT = 32.f;  // log2 units
+constexpr float REG_REDO = 3.0e38f;
+__device__ __forceinline__ bool reg_redo(float sum) { return sum >= 2.9e38f; }
+
+// X holds the logits S (log2; anything in slots of tiles the wave does not have): turns them
+// into E with the potentials pot (by streamed index) as base and the wave's row maxima as shift,
+// and leaves the rows' partials p_w = sh + log2 sum_(its j) E_qj (NEG_BIG for an empty sum) as in
+// flow_chunk.  The potentials enter by one rank-2 MFMA per pair.
 template <int KS, int NRM, int NW>
-__device__ __forceinline__ void reg_sweep(bool online, const f32x4 (&S)[NRM * KS], int nr, const bf16x4* colp,
-                                          const bf16x4* rowp, const float* shift, float* part,
-                                          float* pmax = nullptr) {
+__device__ __forceinline__ void reg_online(f32x4 (&X)[NRM * KS], float (&sh)[NRM], int nr, int n_tiles,
+                                           const float* pot, float* part) {
   const int lane = threadIdx.x & (WAVE - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int g = lane >> 4;
@@ -921,44 +984,112 @@ __device__ __forceinline__ void reg_sweep(bool online, const f32x4 (&S)[NRM * KS
   const bf16x4 zero = {(bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f};
   bf16x4 A[KS];
 #pragma unroll
-  for (int k = 0; k < KS; ++k) A[k] = blk_col_operand(colp, wave + NW * k, lane);
+  for (int k = 0; k < KS; ++k) {
+    const int st = wave + NW * k;
+    const bf16x4 p = split3(st < n_tiles ? pot[st * 16 + (lane & 15)] : NEG_BIG);
+    A[k] = g == 0 ? p : (g == 1 ? one : zero);
+  }
 #pragma unroll
   for (int r = 0; r < NRM; ++r) {
     if (r < nr) {
-      float sh;
-      bf16x4 Bv;
-      if (online) {
-        const bf16x4 b0 = g == 0 ? one : zero;  // row term 0
-        float m = NEG_BIG;
-#pragma unroll
-        for (int k = 0; k < KS; ++k) {
-          const f32x4 x = mfma_rank(A[k], b0, S[r * KS + k]);
-          m = fmaxf(m, fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])));
-        }
-        m = max_groups(m);
-        if (pmax && lane < 16) pmax[(r * 16 + lane) * NW + wave] = m;
-        sh = m > 0.5f * NEG_BIG ? m : 0.f;  // no live entry: the sum is 0 whatever the shift
-        Bv = g == 1 ? split3(-sh) : b0;
-      } else {
-        sh = shift[r * 16 + (lane & 15)];
-        Bv = blk_row_operand(rowp, r, lane);
-      }
-      float e[4 * KS];
-      // software pipelined: the MFMA of pair k + 1 issues before the exponentials of
-      // pair k (two accumulators live), so the exponentials rarely wait on an MFMA
-      f32x4 xc = mfma_rank(A[0], Bv, S[r * KS]);
+      const bf16x4 b0 = g == 0 ? one : zero;  // row term 0
+      float m = NEG_BIG;
 #pragma unroll
       for (int k = 0; k < KS; ++k) {
-        f32x4 xn;
-        if (k + 1 < KS) xn = mfma_rank(A[k + 1], Bv, S[r * KS + k + 1]);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) e[4 * k + q] = fast_exp2(xc[q]);
-        __builtin_amdgcn_sched_barrier(0);
-        if (k + 1 < KS) xc = xn;
+        const f32x4 x = mfma_rank(A[k], b0, X[r * KS + k]);
+        m = fmaxf(m, fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])));
       }
-      const float ss = sum_groups(tree_sum(e));
-      if (lane < 16) part[(r * 16 + lane) * NW + wave] = ss > 0.f ? sh + fast_log2(ss) : NEG_BIG;
+      m = max_groups(m);
+      const bool live = m > 0.5f * NEG_BIG;  // else the sum is 0 whatever the shift
+      const bf16x4 Bv = g == 1 ? split3(live ? -m : 0.f) : b0;
+      sh[r] = live ? m : NEG_BIG;
+      float ss = 0.f;
+#pragma unroll
+      for (int k = 0; k < KS; ++k) {
+        f32x4 x = mfma_rank(A[k], Bv, X[r * KS + k]);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x[q] = fast_exp2(x[q]);
+        ss += (x[0] + x[1]) + (x[2] + x[3]);
+        X[r * KS + k] = x;
+      }
+      ss = sum_groups(ss);
+      // (a NaN passes on; an empty sum is NEG_BIG)
+      if (lane < 16) part[(r * 16 + lane) * NW + wave] = ss <= 0.f ? NEG_BIG : sh[r] + fast_log2(ss);
+    }
+  }
+}
+
+// E and its shift to the common shift lse (local rows) of the sweep that formed E.
+template <int KS, int NRM>
+__device__ __forceinline__ void reg_rescale(f32x4 (&X)[NRM * KS], float (&sh)[NRM], int nr, const float* lse) {
+  const int lane = threadIdx.x & (WAVE - 1);
+#pragma unroll
+  for (int r = 0; r < NRM; ++r) {
+    if (r < nr) {
+      const float l = lse[r * 16 + (lane & 15)], c = fast_exp2(sh[r] - l);
+      sh[r] = l;
+#pragma unroll
+      for (int k = 0; k < KS; ++k)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) X[r * KS + k][q] *= c;
+    }
+  }
+}
+
+// The rows' partial sums sum_(its j) E_qj w_j at the common shift, in flow_chunk's layout.
+// w by streamed index (zero for a masked entry, finite wherever a slot reads).
+template <int KS, int NRM, int NW>
+__device__ __forceinline__ void reg_scaled(const f32x4 (&X)[NRM * KS], int nr, const float* w, float* part) {
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const float* wl = w + wave * 16 + 4 * (lane >> 4);
+  f32x4 a[NRM];
+#pragma unroll
+  for (int k = 0; k < KS; ++k) {
+    const f32x4 wv = *reinterpret_cast<const f32x4*>(wl + NW * 16 * k);
+#pragma unroll
+    for (int r = 0; r < NRM; ++r)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) a[r][q] = k ? __builtin_fmaf(X[r * KS + k][q], wv[q], a[r][q]) : X[r * KS][q] * wv[q];
+  }
+#pragma unroll
+  for (int r = 0; r < NRM; ++r)
+    if (r < nr) {
+      const float ss = sum_groups((a[r][0] + a[r][1]) + (a[r][2] + a[r][3]));
+      if (lane < 16) part[(r * 16 + lane) * NW + wave] = ss;
+    }
+}
+// Sum of the NW partial sums of row q, in wave order.
+template <int NW> __device__ __forceinline__ float reg_sum(const float* part, int q) {
+  float s = 0.f;
+#pragma unroll
+  for (int w4 = 0; w4 < NW; w4 += 4) {
+    const f32x4 v = *reinterpret_cast<const f32x4*>(part + q * NW + w4);
+    s += (v[0] + v[1]) + (v[2] + v[3]);
+  }
+  return s;
+}
+
+// The wave's row maxima (log2, absolute; NEG_BIG where it has no live entry) of the sweep that
+// reg_scaled would make, to pmax in flow_chunk's layout.
+template <int KS, int NRM, int NW>
+__device__ __forceinline__ void reg_row_max(const f32x4 (&X)[NRM * KS], const float (&sh)[NRM], int nr, const float* w,
+                                            float* pmax) {
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int g = lane >> 4;
+#pragma unroll
+  for (int r = 0; r < NRM; ++r) {
+    if (r < nr) {
+      float m = 0.f;  // (entries are not negative)
+#pragma unroll
+      for (int k = 0; k < KS; ++k) {
+        const f32x4 wv = *reinterpret_cast<const f32x4*>(w + (wave + NW * k) * 16 + 4 * g);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) m = fmaxf(m, X[r * KS + k][q] * wv[q]);
+      }
+      m = max_groups(m);
+      if (lane < 16) pmax[(r * 16 + lane) * NW + wave] = m > 0.f ? sh[r] + fast_log2(m) : NEG_BIG;
     }
   }
 }

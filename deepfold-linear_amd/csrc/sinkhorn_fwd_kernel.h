@@ -262,15 +262,15 @@ __device__ __forceinline__ void fwd_resident_output(const SinkFwdArgs& a, int b,
 
 // MODE (compile time, so the plain UOT instantiation carries none of the other
 // modes' code): FWD_UOT, FWD_UOT_HIST (also records the potentials history for the
-// unrolled backward) or FWD_BALANCED (balanced transport, history recorded).  The
-// host picks FWD_BALANCED exactly when a.balanced != 0 and FWD_UOT_HIST when a.hist
-// is given.
+// unrolled backward) or FWD_BALANCED (balanced transport, history recorded), and the
+// same three with the plan in registers (FWD_*_REG).  The host picks a balanced mode
+// exactly when a.balanced != 0 and a history mode when a.hist is given.
 // GEN: the cost may carry position bins or geometry (the host sets it when either
 // is passed); GEN = false compiles no bias code, which keeps the content-only
 // sweeps at their register budget.
-enum FwdMode : int { FWD_UOT = 0, FWD_UOT_HIST = 1, FWD_BALANCED = 2, FWD_UOT_REG = 3 };
+enum FwdMode : int { FWD_UOT = 0, FWD_UOT_HIST = 1, FWD_BALANCED = 2, FWD_UOT_REG = 3, FWD_HIST_REG = 4, FWD_BAL_REG = 5 };
 
-// Register storage of the resident layout (FWD_UOT_REG): a wave holds the logits of
+// Register storage of the resident layout (FWD_*_REG): a wave holds the plan entries of
 // its pairs (resident tile r < nr of the member's stripe, streamed tile wave + 8 k,
 // k < KS) in VGPRs, KS = ceil(n_tiles / 8) rounded up to 2, 4 or 6 and nr at most
 // reg_nrm(KS) (at most 18 pairs per direction, 144 VGPRs for both).
@@ -284,16 +284,16 @@ __host__ __device__ inline bool reg_fits(int N, int G) {
   const int T = (N + 15) / 16, ks = reg_ks(T);
   return ks > 0 && G >= 1 && (T + G - 1) / G <= reg_nrm(ks);
 }
-// Entries of the split-potential arrays: every slot's streamed tile reads inside them.
+// Entries of the multiplier arrays: every slot's streamed tile reads inside them.
 __host__ __device__ inline int reg_cp_rows(int N, int rcap) {
   const int r = 8 * 16 * reg_ks((N + 15) / 16);
   return rcap > r ? rcap : r;
 }
 template <typename T, int DP, bool STREAM, int MODE, bool GEN>
 __global__ void __launch_bounds__(FWD_NT) sinkhorn_fwd_kernel(SinkFwdArgs a) {
-  constexpr bool BAL = MODE == FWD_BALANCED;
-  constexpr bool HIST = MODE == FWD_UOT_HIST || MODE == FWD_BALANCED;
-  constexpr bool REG = !STREAM && MODE == FWD_UOT_REG;
+  constexpr bool BAL = MODE == FWD_BALANCED || MODE == FWD_BAL_REG;
+  constexpr bool HIST = BAL || MODE == FWD_UOT_HIST || MODE == FWD_HIST_REG;
+  constexpr bool REG = !STREAM && (MODE == FWD_UOT_REG || MODE == FWD_HIST_REG || MODE == FWD_BAL_REG);
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ int s_flag, s_tmp, s_local;
   __shared__ unsigned s_du, s_dv;
@@ -330,12 +330,10 @@ __global__ void __launch_bounds__(FWD_NT) sinkhorn_fwd_kernel(SinkFwdArgs a) {
   float* lmu_l = mx2 + loc;     // log mu of my rows
   float* lnu_l = lmu_l + loc;   // log nu of my columns
   float* scratch = lnu_l + loc;
-  // register storage: split parts of u and v (by index) and of -shift of my rows / columns
+  // register storage (scaling form): the multipliers exp2(u - base), exp2(v - base), by index
   const int cpn = REG ? reg_cp_rows(N, rcap) : 0;
-  bf16x4* cpU = reinterpret_cast<bf16x4*>(scratch + sweep_scratch<FWD_NT>());
-  bf16x4* cpV = cpU + cpn;
-  bf16x4* rpR = cpV + cpn;
-  bf16x4* rpC = rpR + loc;
+  float* mulU = scratch + sweep_scratch<FWD_NT>();
+  float* mulV = mulU + cpn;
 
   const int n = mask_setup(a.mask ? a.mask + (size_t)b * N : nullptr, N, valid, &s_tmp);
   const int n_tiles = (n + 15) / 16;
@@ -379,6 +377,13 @@ __global__ void __launch_bounds__(FWD_NT) sinkhorn_fwd_kernel(SinkFwdArgs a) {
   } else {
     stage_rows<T, DP>(QS, Qg, a.sn, n, d, rcap);
     stage_rows<T, DP>(KS, Kg, a.sn, n, d, rcap);
+    // the register tail stages V^T after the last sweep: bring V to L2 meanwhile
+    if constexpr (REG && DP == 32)
+      if (has_v)
+        for (int i = threadIdx.x; i < n; i += FWD_NT) {
+          const float first = to_f32(Vg[(size_t)i * a.sn]), last = to_f32(Vg[(size_t)i * a.sn + d - 1]);
+          asm volatile("" ::"v"(first), "v"(last));
+        }
   }
 
   const float eps = a.eps[h];
@@ -403,13 +408,8 @@ __global__ void __launch_bounds__(FWD_NT) sinkhorn_fwd_kernel(SinkFwdArgs a) {
     vecU[i] = ok ? (a.u_init ? a.u_init[bh * N + i] * LOG2E : 0.f) : NEG_BIG;
     vecV[i] = ok ? (a.v_init ? a.v_init[bh * N + i] * LOG2E : 0.f) : NEG_BIG;
   }
-  if constexpr (REG) {
-    for (int i = threadIdx.x; i < cpn; i += FWD_NT) {  // the same thread wrote vecU[i], vecV[i]
-      cpU[i] = split3(i < rcap ? vecU[i] : NEG_BIG);
-      cpV[i] = split3(i < rcap ? vecV[i] : NEG_BIG);
-    }
-    for (int q = threadIdx.x; q < loc; q += FWD_NT) rpR[q] = rpC[q] = split3(0.f);
-  }
+  if constexpr (REG)
+    for (int i = threadIdx.x; i < 2 * cpn; i += FWD_NT) mulU[i] = 0.f;  // both arrays
   const float w_h = bal ? w_bal : (a.w_dist ? a.w_dist[h] : 0.f);
   const bool use_geo = GEN && (a.x != nullptr) && (w_h != 0.f);
   const bool use_pos = GEN && (a.bins8 != nullptr) && (a.pos_w != nullptr);
@@ -585,7 +585,7 @@ __global__ void __launch_bounds__(FWD_NT) sinkhorn_fwd_kernel(SinkFwdArgs a) {
   // site per update in each instantiation: with two, the compiler outlines them
   // into calls with a stack frame.
   if constexpr (REG) {
-    // ---- register storage: the logits of every wave's pairs stay in VGPRs
+    // ---- register storage: the plan entries of every wave's pairs stay in VGPRs
     bool reg_tail = false;  // the register tail wrote the outputs
     auto reg_loop = [&](auto ksc) __attribute__((always_inline)) -> bool {
       constexpr int KSL = decltype(ksc)::value;
@@ -598,125 +598,205 @@ __global__ void __launch_bounds__(FWD_NT) sinkhorn_fwd_kernel(SinkFwdArgs a) {
         if (threadIdx.x == 0) raise_error(a.err, a.salt, 3u);
         return false;
       }
-      // S[r KSL + k]: row block (i resident, j streamed) and column block (j resident,
-      // i streamed), sc q.k + bias, NEG_BIG where the wave has no tile
-      f32x4 SR[NRM * KSL], SC[NRM * KSL];
+      // X[r KSL + k]: row block (i resident, j streamed) and column block (j resident, i streamed)
+      f32x4 XR[NRM * KSL], XC[NRM * KSL];
+      float shR[NRM], shC[NRM];
+      // bases of the potentials of this wave's streamed entries 64 s + lane
+      constexpr int NB = (16 * KSL + WAVE - 1) / WAVE;
+      float baseV[NB], baseU[NB];
 #pragma unroll
-      for (int r = 0; r < NRM; ++r) {
-#pragma unroll
-        for (int k = 0; k < KSL; ++k) {
-          const int sl = r * KSL + k, st = wave + FWD_NW * k;
-          SR[sl] = SC[sl] = f32x4{NEG_BIG, NEG_BIG, NEG_BIG, NEG_BIG};
-          if (r < nr && st < n_tiles) {
-            const int ri = (t0 + r) * 16 + (lane & 15), si = st * 16 + (lane & 15);
-            typename M::Frag qr, kr, qs, ks;
-            M::load(qr, QS + (size_t)ri * DP, lane);
-            M::load(kr, KS + (size_t)ri * DP, lane);
-            M::load(qs, QS + (size_t)si * DP, lane);
-            M::load(ks, KS + (size_t)si * DP, lane);
-            const f32x4 z = {0.f, 0.f, 0.f, 0.f};
-            const f32x4 xr = M::qk(ks, qr, z);  // [m = j streamed][n = i resident]
-            const f32x4 xc = M::qk(qs, kr, z);  // [m = i streamed][n = j resident]
-            f32x4 br[1] = {z}, bc[1] = {z};
-            if (general) {
-              const int s0[1] = {st * 16 + 4 * g};
-              bias.template quads<false, 1>(ri, s0, br);
-              bias.template quads<true, 1>(ri, s0, bc);
-            }
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              SR[sl][q] = __builtin_fmaf(xr[q], sc, br[0][q]);
-              SC[sl][q] = __builtin_fmaf(xc[q], sc, bc[0][q]);
-            }
-          }
-        }
-      }
+      for (int s = 0; s < NB; ++s) baseU[s] = baseV[s] = 0.f;
       // what the combining thread of local row / column q = threadIdx.x publishes with,
       // loaded once
       const int qc = threadIdx.x, ic = r_lo + qc;
       const bool in_c = qc < nr * 16 && ic < n, ok_c = in_c && valid[ic];
       const float lmu_c = in_c ? lmu_l[qc] : 0.f, lnu_c = in_c ? lnu_l[qc] : 0.f;
-      for (int it = 0; it < a.K_iter; ++it) {
-        // row update: u_i = kappa (log mu_i - LSE_j(L_ij + v_j))
-        {
-          ++phase;
-          const uint32_t tag = salt | phase;
-          bool online = it == 0;
-          if (phase > 1) {
-            float dm;
-            if (!wave_gather<FWD_NW>(xv, n, n_tiles, tag - 1, vecV, valid, a.err, dm, cpV)) s_flagp[phase & 1] = 1;
-            online = online || !(dm <= FIXED_SHIFT_MAX_DELTA);
-          }
-          float* part = scratch + (chunk & 1) * (FWD_NW * SK_RT * 16);
-          ++chunk;
-          reg_sweep<KSL, NRM, FWD_NW>(online, SR, nr, cpV, rpR, lse_r, part);
-          lds_barrier();
-          flow_combine<FWD_NW>(part, nr, lse_r, [&](int q, float l2) {
-            if (in_c) xch_put(xu + ic, kappa * (lmu_c - l2 * LN2), tag, local);
-            rpR[q] = split3(ok_c ? -l2 : 0.f);
-          });
-          // the other waves start polling once the combining threads have published:
-          // earlier polls only load the L2 the publishing stores go through
-          lds_barrier();
-          if (s_flagp[phase & 1]) return false;
-          if (!agree_placement()) return false;
-        }
-        // column update: v_j = kappa (log nu_j - LSE_i(L_ij + u_i))
-        {
-          ++phase;
-          const uint32_t tag = salt | phase;
-          const bool last = it == a.K_iter - 1;
-          float dm;
-          if (!wave_gather<FWD_NW>(xu, n, n_tiles, tag - 1, vecU, valid, a.err, dm, cpU)) s_flagp[phase & 1] = 1;
-          const bool online = it == 0 || !(dm <= FIXED_SHIFT_MAX_DELTA);
-          float* part = scratch + (chunk & 1) * (FWD_NW * SK_RT * 16);
-          ++chunk;
-          reg_sweep<KSL, NRM, FWD_NW>(online, SC, nr, cpU, rpC, lse_c, part);
-          lds_barrier();
-          flow_combine<FWD_NW>(part, nr, lse_c, [&](int q, float l2) {
-            if (in_c) xch_put(xv + ic, kappa * (lnu_c - l2 * LN2), tag, local);
-            rpC[q] = split3(ok_c ? -l2 : 0.f);
-            if (last && ok_c) a.col_lse[bh * N + ic] = l2 * LN2;
-          });
-          lds_barrier();  // as after the row combine
-          if (s_flagp[phase & 1]) return false;
-        }
-      }
-      // ---- Tail from the register logits (where the merge of the output partials
-      // fits the Q and K region, dead after the prologue): the final row sweep (exact
-      // log Z and row maxima) and the output pass, with no QK^T or bias recompute.
-      // (head dim 32: at 64 the output accumulators no longer fit beside the logits)
-      if constexpr (DP == 32) {
+      // Whether the output comes from the register plan (where the merge of the waves'
+      // partials fits the Q and K region, dead after the last sweep; at head dim 64 the output
+      // accumulators no longer fit beside the plan)
       constexpr int NC = DP / 16;
       constexpr int PF = 4 * NC + 3;  // floats of one lane's output partial
-      if ((size_t)FWD_NW * nr * PF * WAVE * sizeof(float) > (size_t)2 * rcap * DP * sizeof(T)) return true;
-      T* VT = QS;  // [DP][Np]; its loads overlap the final sweep
-      stage_rows_t<T, DP>(VT, Vg, a.sn, n, d, Np);
-      {
-        const int fp = (phase + 1) & 1;  // the flag parity of this extra half-iteration
-        float dm;
-        if (!wave_gather<FWD_NW>(xv, n, n_tiles, salt | phase, vecV, valid, a.err, dm, cpV)) s_flagp[fp] = 1;
+      reg_tail = DP == 32 && (size_t)FWD_NW * nr * PF * WAVE * sizeof(float) <= (size_t)2 * rcap * DP * sizeof(T);
+      float* pmax = nullptr;
+      // the logits sc q.k + bias of the wave's pairs, NEG_BIG where it has no tile
+      auto form = [&]() __attribute__((always_inline)) {
+        // opaque copies: nothing of this block is kept in registers across the sweeps
+        int lane_ = lane, t0_ = t0;
+        asm volatile("" : "+v"(lane_), "+v"(t0_));
+        const int g_ = lane_ >> 4;
+        auto block = [&](auto rowc, f32x4(&X)[NRM * KSL]) __attribute__((always_inline)) {
+          constexpr bool ROW = decltype(rowc)::value;
+          uint32_t words[GEN ? NRM * KSL : 1];  // every pair's bins in flight together
+          if constexpr (GEN) {
+#pragma unroll
+            for (int r = 0; r < NRM; ++r)
+#pragma unroll
+              for (int k = 0; k < KSL; ++k) {
+                const int st = wave + FWD_NW * k;
+                words[r * KSL + k] =
+                    r < nr && st < n_tiles
+                        ? bias.template word<!ROW>((t0_ + r) * 16 + (lane_ & 15), st * 16 + 4 * g_) : 0u;
+              }
+          }
+#pragma unroll
+          for (int r = 0; r < NRM; ++r) {
+#pragma unroll
+            for (int k = 0; k < KSL; ++k) {
+              const int sl = r * KSL + k, st = wave + FWD_NW * k;
+              X[sl] = f32x4{NEG_BIG, NEG_BIG, NEG_BIG, NEG_BIG};
+              if (r < nr && st < n_tiles) {
+                const int ri = (t0_ + r) * 16 + (lane_ & 15), si = st * 16 + (lane_ & 15);
+                typename M::Frag fr, fs;
+                M::load(fr, (ROW ? QS : KS) + (size_t)ri * DP, lane_);
+                M::load(fs, (ROW ? KS : QS) + (size_t)si * DP, lane_);
+                const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+                const f32x4 x = M::qk(fs, fr, z);  // [m = streamed][n = resident]
+                f32x4 bb = z;
+                if (general) bb = bias.from_word(words[GEN ? sl : 0], ri, st * 16 + 4 * g_);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) X[sl][q] = __builtin_fmaf(x[q], sc, bb[q]);
+              }
+              if constexpr (GEN) __builtin_amdgcn_sched_barrier(0);  // one pair's bias terms live at a time
+            }
+          }
+        };
+        block(std::integral_constant<bool, true>{}, XR);
+        block(std::integral_constant<bool, false>{}, XC);
+      };
+      // One half-iteration.  ROW: u_i = kappa (log mu_i - LSE_j(L_ij + v_j)) for my rows, else
+      // v_j = kappa (log nu_j - LSE_i(L_ij + u_i)) for my columns.  ONLINE: X holds logits, to be
+      // turned into entries with the present potentials as base, else entries at the rows' common
+      // shifts.  fin: the UOT mode's last row sweep (exact log Z and row maxima), which publishes
+      // nothing.  Returns 0, 1 if the entries have to be formed anew for it (nothing is published
+      // then), or -1 on an expired wait.
+      auto half = [&](auto rowc, auto onl, f32x4(&X)[NRM * KSL], float(&sh)[NRM], float(&base)[NB], float& shift, int it,
+                      bool fin) __attribute__((always_inline)) -> int {
+        constexpr bool ONLINE = decltype(onl)::value;
+        constexpr bool ROW = decltype(rowc)::value;
+        ++phase;
+        const uint32_t tag = salt | phase;
+        float* pot = ROW ? vecV : vecU;
+        float* mul = ROW ? mulV : mulU;
+        float* lse = ROW ? lse_r : lse_c;
+        bool redo = false;
+        if (phase > 1) {  // (the first sweep reads the initial potentials)
+          float dm;
+          if (!wave_gather_scaled<FWD_NW>(ROW ? xv : xu, n, n_tiles, tag - 1, pot, base, mul, valid, a.err, dm))
+            s_flagp[phase & 1] = 1;
+          redo = !(dm <= REG_MAX_DRIFT);
+        }
         float* part = scratch + (chunk & 1) * (FWD_NW * SK_RT * 16);
         ++chunk;
-        float* pmax = reinterpret_cast<float*>(cpU);  // u's parts are dead after the last column sweep
-        reg_sweep<KSL, NRM, FWD_NW>(true, SR, nr, cpV, rpR, lse_r, part, pmax);
+        if constexpr (ONLINE) {
+#pragma unroll
+          for (int s = 0; s < NB; ++s) {
+            const int e = s * WAVE + lane, i = (wave + FWD_NW * (e >> 4)) * 16 + (e & 15);
+            if (e < 16 * KSL && i < n) {
+              base[s] = pot[i];
+              mul[i] = valid[i] ? 1.f : 0.f;
+            }
+          }
+          reg_online<KSL, NRM, FWD_NW>(X, sh, nr, n_tiles, pot, part);
+        } else if (redo) {
+          if (lane < 16)
+            for (int r = 0; r < nr; ++r) part[(r * 16 + lane) * FWD_NW + wave] = REG_REDO;
+        } else {
+          reg_scaled<KSL, NRM, FWD_NW>(X, nr, mul, part);
+        }
+        if (fin) {
+          // the other slot: its partials were combined before the last half-iteration's end
+          pmax = scratch + (chunk & 1) * (FWD_NW * SK_RT * 16);
+          reg_row_max<KSL, NRM, FWD_NW>(X, sh, nr, mul, pmax);
+        }
         lds_barrier();
-        if (s_flagp[fp]) return false;
         if (qc < nr * 16) {
+          float l2;
+          bool pub = true;
+          if constexpr (ONLINE) {
+            l2 = shift = flow_lse<FWD_NW>(part, qc);
+          } else {
+            const float ss = reg_sum<FWD_NW>(part, qc);
+            pub = !reg_redo(ss);
+            l2 = ss <= 0.f ? NEG_BIG : shift + fast_log2(ss);
+          }
+          if (!pub) {
+            atomicOr(&s_flagp[phase & 1], 2);
+          } else {
+            lse[qc] = l2;
+            const float p = kappa * ((ROW ? lmu_c : lnu_c) - l2 * LN2);
+            if (in_c && !fin) {
+              xch_put((ROW ? xu : xv) + ic, p, tag, local);
+              if constexpr (HIST) a.hist[((size_t)(2 * it + (ROW ? 1 : 0)) * a.B * a.H + bh) * N + ic] = ok_c ? p : 0.f;
+            }
+            // the balanced mode ends on a row update, whose words no wave polls
+            if constexpr (BAL && ROW)
+              if (in_c && it == a.K_iter - 1) vecU[ic] = p * LOG2E;
+            if constexpr (!BAL && !ROW)
+              if (it == a.K_iter - 1 && ok_c) a.col_lse[bh * N + ic] = l2 * LN2;
+          }
+        }
+        // the other waves start polling once the combining threads have published:
+        // earlier polls only load the L2 the publishing stores go through
+        lds_barrier();
+        const int f = s_flagp[phase & 1];
+        if (f & 1) return -1;
+        if (f) return 1;
+        return agree_placement() ? 0 : -1;
+      };
+      const std::integral_constant<bool, true> row_c{};
+      const std::integral_constant<bool, false> col_c{};
+      int it = 0;
+      float shiftR = 0.f, shiftC = 0.f;  // common shifts of local row / column qc
+      bool row_turn = !BAL, done = false;
+      const std::integral_constant<bool, true> online_c{};
+      const std::integral_constant<bool, false> scaled_c{};
+      // to the next half-iteration; true after the last one
+      auto advance = [&]() __attribute__((always_inline)) -> bool {
+        if (!BAL && it == a.K_iter) return true;  // the final row sweep
+        if (row_turn == BAL) ++it;                // the iteration's second half
+        row_turn = !row_turn;
+        return it == a.K_iter && (BAL || !reg_tail);
+      };
+      while (true) {
+        form();
+        int st = 0;
+        for (int z = 0; z < 2 && !done; ++z) {
+          st = row_turn ? half(row_c, online_c, XR, shR, baseV, shiftR, it, !BAL && it == a.K_iter)
+                        : half(col_c, online_c, XC, shC, baseU, shiftC, it, false);
+          if (st < 0) return false;
+          done = advance();
+        }
+        if (done) break;
+        reg_rescale<KSL, NRM>(XR, shR, nr, lse_r);
+        reg_rescale<KSL, NRM>(XC, shC, nr, lse_c);
+        while (true) {
+          st = row_turn ? half(row_c, scaled_c, XR, shR, baseV, shiftR, it, !BAL && it == a.K_iter)
+                        : half(col_c, scaled_c, XC, shC, baseU, shiftC, it, false);
+          if (st) break;
+          if (advance()) { done = true; break; }
+        }
+        if (st < 0) return false;
+        if (done) break;
+        // the entries are formed anew and the half-iteration repeated
+        __syncthreads();
+        if (threadIdx.x == 0) s_flagp[phase & 1] = 0;
+        --phase;
+        __syncthreads();
+      }
+      if (!reg_tail) return true;
+      // ---- Tail: P_ij = E_ij w_j exp2(sh_i - lse_i) with the row LSE of the last row sweep;
+      // each wave sums its streamed tiles, the partials meet in LDS and the wave r writes
+      // resident tile r.  No logit or bias is recomputed.
+      if constexpr (DP == 32) {
+        T* VT = QS;  // [DP][Np]: every wave has passed its last sweep
+        if (has_v) stage_rows_t<T, DP>(VT, Vg, a.sn, n, d, Np);
+        if (!BAL && qc < nr * 16) {
           float mm = NEG_BIG;
 #pragma unroll
           for (int w_ = 0; w_ < FWD_NW; ++w_) mm = fmaxf(mm, pmax[qc * FWD_NW + w_]);
           mx2[qc] = mm;
         }
-        flow_combine<FWD_NW>(part, nr, lse_r, [&](int q, float l2) { rpR[q] = split3(ok_c ? -l2 : 0.f); });
         __syncthreads();
-      }
-      // P_ij = exp2(S_ij + v_j - lse_i); each wave sums its streamed tiles, the
-      // partials meet in LDS and the wave r writes resident tile r
-      {
-        bf16x4 A[KSL];
-#pragma unroll
-        for (int k = 0; k < KSL; ++k) A[k] = blk_col_operand(cpV, wave + FWD_NW * k, lane);
         f32x4 oacc[NRM][NC];
         float xc[NRM][3];
 #pragma unroll
@@ -728,15 +808,15 @@ __global__ void __launch_bounds__(FWD_NT) sinkhorn_fwd_kernel(SinkFwdArgs a) {
 #pragma unroll
         for (int r = 0; r < NRM; ++r) {
           if (r < nr) {
-            const bf16x4 Bv = blk_row_operand(rpR, r, lane);
+            const float cr = fast_exp2(shR[r] - lse_r[r * 16 + (lane & 15)]);
 #pragma unroll
             for (int k = 0; k < KSL; ++k) {
               const int st = wave + FWD_NW * k;
               if (st < n_tiles) {
-                const f32x4 x = mfma_rank(A[k], Bv, SR[r * KSL + k]);
+                const f32x4 w = *reinterpret_cast<const f32x4*>(mulV + st * 16 + 4 * g);
                 float pe[4];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) pe[e] = fast_exp2(x[e]);
+                for (int e = 0; e < 4; ++e) pe[e] = XR[r * KSL + k][e] * w[e] * cr;
                 const f32x4* xj = reinterpret_cast<const f32x4*>(xs + 3 * (st * 16 + 4 * g));
                 const f32x4 x0 = xj[0], x1 = xj[1], x2 = xj[2];
                 const float xv[12] = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3],
@@ -745,14 +825,16 @@ __global__ void __launch_bounds__(FWD_NT) sinkhorn_fwd_kernel(SinkFwdArgs a) {
                 for (int e = 0; e < 4; ++e)
 #pragma unroll
                   for (int c = 0; c < 3; ++c) xc[r][c] = __builtin_fmaf(pe[e], xv[3 * e + c], xc[r][c]);
+                if (has_v) {
 #pragma unroll
-                for (int c = 0; c < NC; ++c)
-                  oacc[r][c] = reg_pv<T>(pe, VT + (size_t)(c * 16 + (lane & 15)) * Np + st * 16 + 4 * g, oacc[r][c]);
+                  for (int c = 0; c < NC; ++c)
+                    oacc[r][c] = reg_pv<T>(pe, VT + (size_t)(c * 16 + (lane & 15)) * Np + st * 16 + 4 * g, oacc[r][c]);
+                }
               }
             }
           }
         }
-        __syncthreads();  // V^T and the split parts are read
+        __syncthreads();  // V^T is read
         float* mg = reinterpret_cast<float*>(QS);
 #pragma unroll
         for (int r = 0; r < NRM; ++r) {
@@ -783,10 +865,8 @@ __global__ void __launch_bounds__(FWD_NT) sinkhorn_fwd_kernel(SinkFwdArgs a) {
             for (int c = 0; c < 3; ++c) x3[c] += src[(4 * NC + c) * WAVE];
           }
           fwd_write_tile<T, DP>(a, b, h, t0 + r, n, valid, lse_r + r * 16, mx2 + r * 16, vecU, vecV, o, x3[0], x3[1],
-                                x3[2], Gg, lane, false);
+                                x3[2], Gg, lane, bal);
         }
-      }
-      reg_tail = true;
       }
       return true;
     };
@@ -836,8 +916,8 @@ __global__ void __launch_bounds__(FWD_NT) sinkhorn_fwd_kernel(SinkFwdArgs a) {
   const int g = lane >> 4;
   constexpr int NC = DP / 16;
   if constexpr (!STREAM) {
-    // register storage: the sweep scratch and the split-potential arrays are free now
-    const int free_floats = REG ? sweep_scratch<FWD_NT>() + (2 * cpn + 2 * loc) * 2 : 0;
+    // register storage: the sweep scratch and the multiplier arrays are free now
+    const int free_floats = REG ? sweep_scratch<FWD_NT>() + 2 * cpn : 0;
     fwd_resident_output<T, DP>(a, b, h, n, n_tiles, Np, t0, nr, valid, QS, KS, vecU, vecV, xs, lse2, mx2, sc, bias,
                                general, bal, has_v, Qg, Vg, Gg, scratch, free_floats);
   } else {
@@ -948,7 +1028,7 @@ inline size_t sinkhorn_fwd_lds_bytes_t(int N, int DP, int elem, int G, bool stre
     bytes += (2 * rcap + 3 * Np) * 4;     // vecU, vecV, xs
     bytes += 5 * loc * 4;                 // lse_r, lse_c, mx2, lmu_l, lnu_l
     bytes += (size_t)sweep_scratch<FWD_NT>() * 4;
-    if (reg) bytes += (2 * (size_t)reg_cp_rows(N, (int)rcap) + 2 * loc) * 8;  // cpU, cpV, rpR, rpC
+    if (reg) bytes += 2 * (size_t)reg_cp_rows(N, (int)rcap) * 4;  // mulU, mulV
   }
   return bytes;
 }
@@ -971,7 +1051,7 @@ static hipError_t launch_fwd_t(const SinkFwdArgs& a, size_t lds, hipStream_t str
 template <bool STREAM, int MODE, bool GEN>
 hipError_t launch_fwd_dt(const SinkFwdArgs& a, bool bf16_in, int DP, size_t lds, hipStream_t stream, bool coop) {
   if (bf16_in) {
-    if constexpr (MODE == FWD_BALANCED) return hipErrorInvalidValue;  // the balanced transport is fp32 only
+    if constexpr (MODE == FWD_BALANCED || MODE == FWD_BAL_REG) return hipErrorInvalidValue;  // the balanced transport is fp32 only
     else {
       if (DP == 32) return launch_fwd_t<bf16, 32, STREAM, MODE, GEN>(a, lds, stream, coop);
       if (DP == 64) return launch_fwd_t<bf16, 64, STREAM, MODE, GEN>(a, lds, stream, coop);
@@ -979,18 +1059,6 @@ hipError_t launch_fwd_dt(const SinkFwdArgs& a, bool bf16_in, int DP, size_t lds,
   } else {
     if (DP == 32) return launch_fwd_t<float, 32, STREAM, MODE, GEN>(a, lds, stream, coop);
     if (DP == 64) return launch_fwd_t<float, 64, STREAM, MODE, GEN>(a, lds, stream, coop);
-  }
-  return hipErrorInvalidValue;
-}
-
-template <bool GEN>
-hipError_t launch_fwd_reg_dt(const SinkFwdArgs& a, bool bf16_in, int DP, size_t lds, hipStream_t stream, bool coop) {
-  if (bf16_in) {
-    if (DP == 32) return launch_fwd_t<bf16, 32, false, FWD_UOT_REG, GEN>(a, lds, stream, coop);
-    if (DP == 64) return launch_fwd_t<bf16, 64, false, FWD_UOT_REG, GEN>(a, lds, stream, coop);
-  } else {
-    if (DP == 32) return launch_fwd_t<float, 32, false, FWD_UOT_REG, GEN>(a, lds, stream, coop);
-    if (DP == 64) return launch_fwd_t<float, 64, false, FWD_UOT_REG, GEN>(a, lds, stream, coop);
   }
   return hipErrorInvalidValue;
 }

@@ -1,0 +1,99 @@
+"""Register storage in scaling form: potentials that move further than the plan entries'
+bases allow (the workgroup forms its entries anew), few iterations (the entries' common
+shift not yet taken), and the edges of the register tiles, for the plain, the history and
+the balanced forward.  Float64 oracles; normwise bar 1e-4 (fp32 inputs)."""
+
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from conftest import assert_close_rel
+from oracle import balanced_transport as bt
+from oracle import sinkhorn as ref
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+MAX_DRIFT = 32 * math.log(2.0)  # nats
+
+
+def _uot(B, H, N, d, K, seed, v_scale, lengths):
+    g = torch.Generator().manual_seed(seed)
+    rn = lambda *s: torch.randn(*s, generator=g)
+    t = dict(Q=rn(B, H, N, d), K=rn(B, H, N, d), V=rn(B, H, N, d), G=rn(B, H, N, d), x_res=rn(B, N, 3),
+             pos_weight=torch.zeros(H, 68), eps=torch.linspace(0.3, 1.0, H), w_dist=torch.zeros(H),
+             log_v_init=v_scale * rn(B, H, N), log_u_init=torch.zeros(B, H, N))
+    mask = torch.zeros(B, N)
+    lmu, lnu = torch.zeros(B, H, N), torch.zeros(B, H, N)
+    for b, n in enumerate(lengths):
+        mask[b, :n] = 1
+        lmu[b, :, :n] = torch.log_softmax(rn(H, n), -1)
+        lnu[b, :, :n] = torch.log_softmax(rn(H, n), -1)
+    t["log_v_init"] *= mask[:, None, :]
+    t.update(log_mu=lmu, log_nu=lnu, mask=mask)
+    return t
+
+
+@pytest.mark.parametrize("unrolled", [False, True])
+@pytest.mark.parametrize("B,H,N,d,K,v_scale,lengths", [
+    (1, 4, 256, 32, 1, 0.5, [256]),     # the tail follows the sweeps that formed the entries
+    (1, 4, 250, 32, 2, 40.0, [250]),    # initial potentials far from the first update: formed anew
+    (2, 8, 300, 32, 5, 40.0, [300, 161]),
+    (2, 8, 500, 24, 3, 0.5, [497, 16]),  # a member without a second tile, and one without any
+    (1, 8, 200, 64, 3, 40.0, [200]),    # head dim 64: the recomputing tail
+])
+def test_register_forward(B, H, N, d, K, v_scale, lengths, unrolled):
+    from deepfold_amd import flash_sinkhorn_attn
+
+    print(f"case B{B} H{H} N{N} d{d} K{K} v{v_scale} unrolled={unrolled}", flush=True)
+    t = _uot(B, H, N, d, K, N + K, v_scale, lengths)
+    c = {k: v.to(DEV) for k, v in t.items()}
+    out = flash_sinkhorn_attn(c["Q"], c["K"], c["V"], c["G"], c["x_res"], c["pos_weight"], None, c["eps"], None,
+                              c["log_mu"], c["log_nu"], K_iter=K, log_u_init=c["log_u_init"],
+                              log_v_init=c["log_v_init"], mask=c["mask"],
+                              ift_mode="unrolled" if unrolled else "reference")
+    n64 = {k: v.double().numpy() for k, v in t.items()}
+    args = dict(Q=n64["Q"], K=n64["K"], V=n64["V"], G=n64["G"], x_res=n64["x_res"], pos_weight=n64["pos_weight"],
+                pos_bins=None, eps=n64["eps"], w_dist=n64["w_dist"], log_mu=n64["log_mu"], log_nu=n64["log_nu"],
+                log_u_init=n64["log_u_init"], log_v_init=n64["log_v_init"], mask=n64["mask"])
+    want = ref.forward(K_iter=K, **args)
+    if v_scale > 1:  # the case moves some potential past the bound
+        one = ref.forward(K_iter=1, **args)
+        assert np.max(np.abs(one["log_v"] - n64["log_v_init"])) > MAX_DRIFT
+    valid = t["mask"].numpy()[:, None, :, None]
+    for name, got in zip(("o_flat", "x_centroid", "log_u", "log_v"), out):
+        w = want[name] * (valid if name == "x_centroid" else 1.0)
+        assert_close_rel(got.detach().cpu().double().numpy(), w, 1e-4, name)
+
+
+@pytest.mark.parametrize("B,H,N,d,K,eps,lengths", [
+    (1, 16, 256, 32, 1, 0.5, None),
+    (1, 8, 250, 32, 6, 0.01, None),          # logits of +-100 nats: formed anew
+    (2, 16, 384, 32, 4, 0.02, [384, 200]),   # three tiles a member
+    (1, 8, 130, 64, 5, 0.02, [117]),         # the recomputing tail
+])
+def test_register_balanced(B, H, N, d, K, eps, lengths):
+    from deepfold_amd import balanced_sinkhorn_transport_dual
+
+    print(f"case B{B} H{H} N{N} d{d} K{K} eps{eps}", flush=True)
+    g = torch.Generator().manual_seed(N + K)
+    unit = lambda t: t / t.norm(dim=-1, keepdim=True)
+    Q, Kk = unit(torch.randn(B, H, N, d, generator=g)), unit(torch.randn(B, H, N, d, generator=g))
+    Kk[:, :, 0] = Q[:, :, 0]  # one aligned pair: a column potential far from the others
+    x, V = 3 * torch.randn(B, N, 3, generator=g), torch.randn(B, H, N, d, generator=g)
+    e, al, r = torch.full((H,), eps), torch.full((H,), -1.0), torch.full((H,), 10.0)
+    mask = None
+    if lengths is not None:
+        mask = torch.zeros(B, N)
+        for b, n in enumerate(lengths):
+            mask[b, :n] = 1
+    dev = lambda t: None if t is None else t.to(DEV)
+    xc, hc = balanced_sinkhorn_transport_dual(dev(Q), dev(Kk), dev(x), dev(V), dev(e), dev(al), dev(r), K_iter=K,
+                                              mask=dev(mask))
+    f = lambda t: None if t is None else t.double()
+    wx, wh = bt.balanced_transport_dual(f(Q), f(Kk), f(x), f(V), f(e), f(al), f(r), K_iter=K, mask=f(mask))
+    # sharp plans: the logits' fp32 rounding (2^-24 of 100 nats) enters every entry
+    tol = 1e-4
+    assert_close_rel(xc.cpu().double().numpy(), wx.numpy(), tol, "x_centroid")
+    assert_close_rel(hc.cpu().double().numpy(), wh.numpy(), tol, "h_centroid")
