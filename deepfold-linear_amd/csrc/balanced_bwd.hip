@@ -35,6 +35,7 @@
 // element, and no cross-workgroup partial sums of N x d products are needed.
 #include <type_traits>
 
+#include "scaled_bwd.h"
 #include "sinkhorn_bwd_kernel.h"
 
 namespace dfl {
@@ -53,6 +54,7 @@ template <int DP>
 __global__ void __launch_bounds__(256) balanced_prep_kernel(BalPrepArgs p) {
   const int N = p.N, d = p.d;
   const int Np = ((N + 31) / 32) * 32;
+  sb_clear_steps(p.steps, p.B * p.H, N, p.K);
   const size_t e = (size_t)blockIdx.x * 256 + threadIdx.x;
   const size_t row = e / DP;
   const int c = (int)(e % DP);
@@ -114,8 +116,9 @@ __global__ void __launch_bounds__(256) balanced_finalize_kernel(BalBwdArgs a, fl
   }
 }
 
+// The general sweeps of one workgroup.
 template <int DP>
-__global__ void __launch_bounds__(BAL_NT) balanced_bwd_kernel(BalBwdArgs a) {
+__device__ __forceinline__ void balanced_general(const BalBwdArgs& a) {
   using M = Mfma<float, DP>;
   constexpr int NC = DP / 16;
   constexpr int NW = BAL_NW;
@@ -484,6 +487,18 @@ __global__ void __launch_bounds__(BAL_NT) balanced_bwd_kernel(BalBwdArgs a) {
   }
 }
 
+template <int DP>
+__global__ void __launch_bounds__(BAL_NT) balanced_bwd_kernel(BalBwdArgs a) {
+  balanced_general<DP>(a);
+}
+// Register form (scaled_bwd.h); the general sweeps are a call, so that they cost its sweeps no registers.
+__device__ __attribute__((noinline)) void balanced_general_call(BalBwdArgs a) { balanced_general<32>(a); }
+__global__ void __launch_bounds__(SB_NT) balanced_scaled_kernel(BalBwdArgs a) {
+  scaled_bwd<float, true>(a, [](const BalBwdArgs& x) { balanced_general_call(x); });
+}
+
+size_t scaled_step_words(int N) { return sb_step_words(N); }
+
 size_t balanced_bwd_lds_bytes(int N, int DP) {
   (void)DP;
   const size_t Np = ((N + 31) / 32) * 32;
@@ -508,9 +523,9 @@ hipError_t launch_balanced_prep(const BalPrepArgs& p, int DP, hipStream_t stream
   return hipGetLastError();
 }
 
-template <int DP>
-static hipError_t launch_bal_t(const BalBwdArgs& a, size_t lds, hipStream_t stream, bool coop) {
-  auto kern = balanced_bwd_kernel<DP>;
+constexpr size_t BAL_STATIC = 2048;  // static LDS of the register form and the general sweeps, rounded up
+static hipError_t launch_bal_k(void (*kern)(BalBwdArgs), const BalBwdArgs& a, size_t lds, hipStream_t stream,
+                               bool coop) {
   hipError_t e = set_lds_limit((const void*)kern, lds);
   if (e != hipSuccess) return e;
   dim3 grid(grid_blocks(a.B * a.H, a.G)), block(BAL_NT);
@@ -523,9 +538,12 @@ static hipError_t launch_bal_t(const BalBwdArgs& a, size_t lds, hipStream_t stre
   return hipGetLastError();
 }
 
-hipError_t launch_balanced_bwd(const BalBwdArgs& a, int DP, size_t lds, hipStream_t stream, bool coop) {
-  if (DP == 32) return launch_bal_t<32>(a, lds, stream, coop);
-  if (DP == 64) return launch_bal_t<64>(a, lds, stream, coop);
+// The register form where the stripes and the iterations' vectors fit (limit: LDS of a workgroup).
+hipError_t launch_balanced_bwd(const BalBwdArgs& a, int DP, size_t lds, size_t limit, hipStream_t stream, bool coop) {
+  if (sb_fits(a.N, DP, a.G, a.K, true, limit - BAL_STATIC))
+    return launch_bal_k(balanced_scaled_kernel, a, std::max(lds, sb_lds_bytes(a.N, a.G, a.K, true)), stream, coop);
+  if (DP == 32) return launch_bal_k(balanced_bwd_kernel<32>, a, lds, stream, coop);
+  if (DP == 64) return launch_bal_k(balanced_bwd_kernel<64>, a, lds, stream, coop);
   return hipErrorInvalidValue;
 }
 

@@ -62,13 +62,15 @@ hipError_t launch_fill_u64(uint64_t* p, size_t n, hipStream_t stream);
 size_t balanced_bwd_lds_bytes(int N, int DP);
 int balanced_max_tiles(int DP);
 hipError_t launch_balanced_prep(const BalPrepArgs& p, int DP, hipStream_t stream);
-hipError_t launch_balanced_bwd(const BalBwdArgs& a, int DP, size_t lds, hipStream_t stream, bool coop);
+hipError_t launch_balanced_bwd(const BalBwdArgs& a, int DP, size_t lds, size_t limit, hipStream_t stream, bool coop);
+size_t scaled_step_words(int N);
 hipError_t launch_balanced_finalize(const BalBwdArgs& a, float* dx, float* dalpha, float* dr, hipStream_t stream);
 size_t unrolled_bwd_lds_bytes(int N, int DP, int elem, int ops);
 int unrolled_operand_mode(int N, int DP, int elem, size_t limit);
 int unrolled_max_tiles(int DP);
 hipError_t launch_unrolled_prep(const UnrPrepArgs& p, bool bf16_in, int DP, hipStream_t stream);
-hipError_t launch_unrolled_bwd(const UnrBwdArgs& a, bool bf16_in, int DP, size_t lds, hipStream_t stream, bool coop,
+hipError_t launch_unrolled_bwd(const UnrBwdArgs& a, bool bf16_in, int DP, size_t lds, size_t limit,
+                               hipStream_t stream, bool coop,
                                int ops);
 hipError_t launch_unrolled_finalize(const UnrBwdArgs& a, float* dx, float* dpw, float* dw, hipStream_t stream);
 }  // namespace dfl
@@ -577,7 +579,7 @@ int run_fwd(dfl::SinkFwdArgs& a, bool bf16, int DP, int storage, const FwdScratc
 // Balanced transport workspace: the forward's (header, exchange words, stream
 // region), or the backward's prepared operands and partials if larger.
 struct BalWs {
-  size_t qp, kp, qt, kt, vp, gp, gt, dcoef, gxs, xs, dx_part, ar_part, total;
+  size_t steps, qp, kp, qt, kt, vp, gp, gt, dcoef, gxs, xs, dx_part, ar_part, total;
 };
 BalWs bal_ws_layout(int B, int H, int N, int d) {
   auto r256 = [](size_t x) { return (x + 255) / 256 * 256; };
@@ -586,7 +588,8 @@ BalWs bal_ws_layout(int B, int H, int N, int d) {
   const int G = group_size(B, H, N);
   const size_t op = r256((size_t)B * H * np * DP * 4);
   BalWs w;
-  w.qp = r256(WS_HEADER + xch_words(B, H, N) * 8);
+  w.steps = WS_HEADER + xch_words(B, H, N) * 8;
+  w.qp = r256(w.steps + (size_t)B * H * dfl::scaled_step_words(N) * 8);
   w.kp = w.qp + op;
   w.qt = w.kp + op;
   w.kt = w.qt + op;
@@ -615,7 +618,7 @@ size_t bal_fwd_need(int B, int H, int N, int d, int storage) {
 // Unrolled UOT backward workspace: header, exchange words, fp32 operand copies
 // (Q, K, V, gO rows; Q, K, gO transposed), vectors and partials.
 struct UnrWs {
-  size_t qp, kp, qt, kt, vp, gp, gt, dcoef, gxs, xs, dx_part, dpw_part, dw_part, total;
+  size_t steps, qp, kp, qt, kt, vp, gp, gt, dcoef, gxs, xs, dx_part, dpw_part, dw_part, total;
 };
 UnrWs unr_ws_layout(int B, int H, int N, int d) {
   auto r256 = [](size_t x) { return (x + 255) / 256 * 256; };
@@ -624,7 +627,8 @@ UnrWs unr_ws_layout(int B, int H, int N, int d) {
   const int G = group_size(B, H, N);
   const size_t op = r256((size_t)B * H * np * DP * 4);
   UnrWs w;
-  w.qp = r256(WS_HEADER + xch_words(B, H, N) * 8);
+  w.steps = WS_HEADER + xch_words(B, H, N) * 8;
+  w.qp = r256(w.steps + (size_t)B * H * dfl::scaled_step_words(N) * 8);
   w.kp = w.qp + op;
   w.qt = w.kp + op;
   w.kt = w.qt + op;
@@ -1154,6 +1158,7 @@ int dfl_balanced_bwd(const dfl_balanced_bwd_params* p, void* workspace, size_t w
   pr.qp = F(L.qp); pr.kp = F(L.kp); pr.qt = F(L.qt); pr.kt = F(L.kt);
   pr.vp = has_h ? F(L.vp) : nullptr; pr.gp = has_h ? F(L.gp) : nullptr; pr.gt = has_h ? F(L.gt) : nullptr;
   pr.dcoef = F(L.dcoef); pr.gxs = F(L.gxs); pr.xs = F(L.xs);
+  pr.steps = reinterpret_cast<uint64_t*>(ws + L.steps); pr.K = p->K_iter;
   hipError_t e = dfl::launch_balanced_prep(pr, DP, (hipStream_t)stream);
   if (e != hipSuccess) return hip_fail(e, "balanced backward prep launch");
   dfl::BalBwdArgs a;
@@ -1165,11 +1170,12 @@ int dfl_balanced_bwd(const dfl_balanced_bwd_params* p, void* workspace, size_t w
   a.dq = p->dq; a.dk = p->dk; a.dv = p->dv; a.dx_part = F(L.dx_part); a.ar_part = F(L.ar_part);
   a.err = err_ref(ws);
   a.xch = reinterpret_cast<uint64_t*>(ws + WS_HEADER);
+  a.steps = reinterpret_cast<uint64_t*>(ws + L.steps);
   a.G = G;
   if (int rc = refuse_capture(stream, "dfl_balanced_bwd")) return rc;
   if (int rc = acquire_salt(ws, WS_HEADER + xch_words(p->B, p->H, p->N) * 8, stream, &a.salt))
     return hip_fail((hipError_t)rc, "workspace clear launch");
-  e = dfl::launch_balanced_bwd(a, DP, lds, (hipStream_t)stream, coop_launch(G, a.B * a.H));
+  e = dfl::launch_balanced_bwd(a, DP, lds, LDS_LIMIT, (hipStream_t)stream, coop_launch(G, a.B * a.H));
   if (e != hipSuccess) return hip_fail(e, "balanced backward launch");
   e = dfl::launch_balanced_finalize(a, p->dx_res, p->dalpha_h, p->dr_h, (hipStream_t)stream);
   if (e != hipSuccess) return hip_fail(e, "balanced backward finalize launch");
@@ -1220,6 +1226,7 @@ int dfl_sinkhorn_unrolled_bwd(const dfl_sinkhorn_unrolled_bwd_params* p, void* w
   pr.qp = F(L.qp); pr.kp = F(L.kp); pr.qt = F(L.qt); pr.kt = F(L.kt);
   pr.vp = F(L.vp); pr.gp = F(L.gp); pr.gt = F(L.gt);
   pr.dcoef = F(L.dcoef); pr.gxs = F(L.gxs); pr.xs = F(L.xs); pr.dg = p->dg;
+  pr.steps = reinterpret_cast<uint64_t*>(ws + L.steps); pr.K = p->K_iter;
   hipError_t e = dfl::launch_unrolled_prep(pr, p->dtype == DFL_BF16, DP, (hipStream_t)stream);
   if (e != hipSuccess) return hip_fail(e, "unrolled backward prep launch");
   dfl::UnrBwdArgs a;
@@ -1239,11 +1246,12 @@ int dfl_sinkhorn_unrolled_bwd(const dfl_sinkhorn_unrolled_bwd_params* p, void* w
   a.dx_part = F(L.dx_part); a.dpw_part = F(L.dpw_part); a.dw_part = F(L.dw_part);
   a.err = err_ref(ws);
   a.xch = reinterpret_cast<uint64_t*>(ws + WS_HEADER);
+  a.steps = reinterpret_cast<uint64_t*>(ws + L.steps);
   a.G = G;
   if (int rc = refuse_capture(stream, "dfl_sinkhorn_unrolled_bwd")) return rc;
   if (int rc = acquire_salt(ws, WS_HEADER + xch_words(p->B, p->H, p->N) * 8, stream, &a.salt))
     return hip_fail((hipError_t)rc, "workspace clear launch");
-  e = dfl::launch_unrolled_bwd(a, p->dtype == DFL_BF16, DP, lds, (hipStream_t)stream, coop_launch(G, a.B * a.H),
+  e = dfl::launch_unrolled_bwd(a, p->dtype == DFL_BF16, DP, lds, LDS_LIMIT, (hipStream_t)stream, coop_launch(G, a.B * a.H),
                                ops);
   if (e != hipSuccess) return hip_fail(e, "unrolled backward launch");
   e = dfl::launch_unrolled_finalize(a, p->x_res ? p->dx_res : nullptr, p->dpos_weight, p->dw_dist,

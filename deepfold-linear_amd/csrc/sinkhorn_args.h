@@ -148,6 +148,7 @@ struct BalBwdArgs {
   float* dx_part;      // (B,H,N,3) per-head partials
   float* ar_part;      // (B*H*G, 2) per-workgroup d alpha, d r partials
   uint64_t* xch;       // B*H*2*Np exchange words
+  uint64_t* steps;     // sb_step_words(N) per (b,h): the register form's kept exchange words
   ErrRef err;
   int G;
   uint32_t salt;
@@ -167,7 +168,7 @@ struct UnrBwdArgs {
   const float* log_z;
   const float* v_init;   // (B,H,N) or null (zeros)
   const uint8_t* bins8;  // padded uint8 bins [B][Np][Np] (bins8_kernel) or null
-  const uint8_t* bins8t; // transposed copy (unused here)
+  const uint8_t* bins8t; // transposed copy
   const float* pos_w;    // (H,68) or null
   const float* w_dist;   // (H,) or null
   int has_geo;           // geometry term present (x given and w_dist given)
@@ -191,6 +192,7 @@ struct UnrBwdArgs {
   float* dpw_part;       // (B*H*G, 68)
   float* dw_part;        // (B*H*G)
   uint64_t* xch;
+  uint64_t* steps;       // sb_step_words(N) per (b,h): the register form's kept exchange words
   ErrRef err;
   int G;
   uint32_t salt;
@@ -214,6 +216,8 @@ struct UnrPrepArgs {
   float* vp; float* gp; float* gt;
   float* dcoef; float* gxs; float* xs;
   void* dg;              // (B,H,N,d) in the input type, or null (no gate)
+  uint64_t* steps;       // kept exchange words of the register form, cleared for K iterations
+  int K;
 };
 
 struct BalPrepArgs {
@@ -231,6 +235,8 @@ struct BalPrepArgs {
   float* qp; float* kp; float* qt; float* kt;
   float* vp; float* gp; float* gt;  // null without grad_hc
   float* dcoef; float* gxs; float* xs;
+  uint64_t* steps;     // kept exchange words of the register form, cleared for K iterations
+  int K;
 };
 
 // Zero-padded operand copies for stream mode, written by sinkhorn_pad_kernel.

@@ -681,20 +681,17 @@ __device__ __forceinline__ bf16x4 blk_row_operand(const bf16x4* parts, int tile,
 // (lane: rows 4(l/16) + e, V column l % 16).  vt: V^T row (c0 + l%16) at column
 // st*16 + 4(l/16).  bf16: P as a hi + lo pair of bf16 A operands (two
 // 16x16x16 MFMAs on the same V operand); fp32: four 16x16x4 steps.
-template <typename T> __device__ __forceinline__ f32x4 reg_pv(const float (&p)[4], const T* vt, f32x4 acc);
-template <> __device__ __forceinline__ f32x4 reg_pv<bf16>(const float (&p)[4], const bf16* vt, f32x4 acc) {
+__device__ __forceinline__ f32x4 reg_pv(const float (&p)[4], const bf16x4& v, f32x4 acc) {
   bf16x4 hi, lo;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     hi[e] = (bf16)p[e];
     lo[e] = (bf16)(p[e] - (float)hi[e]);
   }
-  const bf16x4 v = *reinterpret_cast<const bf16x4*>(vt);
   acc = mfma_rank(hi, v, acc);
   return mfma_rank(lo, v, acc);
 }
-template <> __device__ __forceinline__ f32x4 reg_pv<float>(const float (&p)[4], const float* vt, f32x4 acc) {
-  const f32x4 v = *reinterpret_cast<const f32x4*>(vt);
+__device__ __forceinline__ f32x4 reg_pv(const float (&p)[4], const f32x4& v, f32x4 acc) {
 #pragma unroll
   for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(p[e], v[e], acc, 0, 0, 0);
   return acc;
@@ -711,9 +708,8 @@ template <> __device__ __forceinline__ f32x4 reg_pv<float>(const float (&p)[4], 
 // with at most 4 resident tiles (2 with a bias).
 
 // Polls the words of this wave's streamed tiles (entries i < n) until they carry `tag`,
-// hands each entry and its new value word * log2 e (NEG_BIG for a masked entry, and at least
-// NEG_BIG) to take(s, i, value, valid), s = 0, 1, ... the lane's entries in order, which returns
-// its |change|, and sets dmax, in every lane, to the largest of them over the wave.  MAXW: most
+// hands each entry's value to take(s, i, value, valid), s = 0, 1, ... the lane's entries in
+// order, which returns its |change|, and sets dmax, in every lane, to the largest of them over the wave.  MAXW: most
 // entries of a lane (a wave's words over 64), 0 for any number (s is then 0 or 1).  Returns false, uniformly over the wave, if a wait
 // expired (then the error has been raised).
 template <int NW, int MAXW, typename Take>
@@ -735,8 +731,7 @@ __device__ __forceinline__ bool wave_poll(const uint64_t* buf, int n, int n_tile
     }
     ok = poll_words<W>(buf, idx, tag, err, [&](int k, uint64_t w) {
       const int i = idx[k];
-      const float nv = __uint_as_float((uint32_t)(w >> 32)) * LOG2E;
-      dm = fmaxf(dm, valid[i] ? take(k, i, nv < NEG_BIG ? NEG_BIG : nv, true) : take(k, i, NEG_BIG, false));
+      dm = fmaxf(dm, take(k, i, __uint_as_float((uint32_t)(w >> 32)), valid[i] != 0));
     });
     ok = wave_max_u32(ok ? 0u : 1u) == 0u;
   };
@@ -749,24 +744,31 @@ __device__ __forceinline__ bool wave_poll(const uint64_t* buf, int n, int n_tile
   dmax = __uint_as_float(wave_max_u32(dm == dm ? __float_as_uint(dm) : 0x7f800000u));
   return ok;
 }
-// wave_poll into dst[i]; dmax is the largest |change| of a valid entry.
+// An exchanged potential in log2 units (NEG_BIG for a masked entry, and at least NEG_BIG).
+__device__ __forceinline__ float pot2(float v, bool ok) {
+  const float nv = v * LOG2E;
+  return !ok || nv < NEG_BIG ? NEG_BIG : nv;
+}
+// wave_poll of potentials into dst[i] (pot2); dmax is the largest |change| of a valid entry.
 template <int NW>
 __device__ __forceinline__ bool wave_gather(const uint64_t* buf, int n, int n_tiles, uint32_t tag, float* dst,
                                             const unsigned char* valid, ErrRef err, float& dmax) {
-  return wave_poll<NW, 0>(buf, n, n_tiles, tag, valid, err, dmax, [&](int, int i, float nv, bool ok) {
+  return wave_poll<NW, 0>(buf, n, n_tiles, tag, valid, err, dmax, [&](int, int i, float v, bool ok) {
+    const float nv = pot2(v, ok);
     const float d = ok ? fabsf(nv - dst[i]) : 0.f;
     dst[i] = nv;
     return d;
   });
 }
-// wave_poll into dst[i] and the multipliers w[i] = exp2(dst[i] - base) of scaling form (0 for a
+// wave_poll of potentials into dst[i] and the multipliers w[i] = exp2(dst[i] - base) of scaling form (0 for a
 // masked entry), with the bases in registers: base[s] of entry 64 s + lane of the wave's words
 // (the wave's tiles in order, 16 entries each).  dmax is the largest |dst - base| of a valid entry.
 template <int NW, int NB>
 __device__ __forceinline__ bool wave_gather_scaled(const uint64_t* buf, int n, int n_tiles, uint32_t tag, float* dst,
                                                    const float (&base)[NB], float* w, const unsigned char* valid,
                                                    ErrRef err, float& dmax) {
-  return wave_poll<NW, NB>(buf, n, n_tiles, tag, valid, err, dmax, [&](int s, int i, float nv, bool ok) {
+  return wave_poll<NW, NB>(buf, n, n_tiles, tag, valid, err, dmax, [&](int s, int i, float v, bool ok) {
+    const float nv = pot2(v, ok);
     const float d = nv - base[s];
     dst[i] = nv;
     w[i] = ok ? fast_exp2(d) : 0.f;
@@ -1092,6 +1094,11 @@ __device__ __forceinline__ void reg_row_max(const f32x4 (&X)[NRM * KS], const fl
       if (lane < 16) pmax[(r * 16 + lane) * NW + wave] = m > 0.f ? sh[r] + fast_log2(m) : NEG_BIG;
     }
   }
+}
+
+template <typename T> using reg_vt = std::conditional_t<sizeof(T) == 2, bf16x4, f32x4>;
+template <typename T> __device__ __forceinline__ f32x4 reg_pv(const float (&p)[4], const T* vt, f32x4 acc) {
+  return reg_pv(p, *reinterpret_cast<const reg_vt<T>*>(vt), acc);
 }
 
 // Exchange-placement agreement of a group.  At the start of a launch every member

@@ -28,6 +28,7 @@
 // 2K + 2 sweeps, at most two exponentials per element each.
 #include <type_traits>
 
+#include "scaled_bwd.h"
 #include "sinkhorn_bwd_kernel.h"
 
 namespace dfl {
@@ -45,6 +46,7 @@ template <typename T, int DP>
 __global__ void __launch_bounds__(256) unrolled_prep_kernel(UnrPrepArgs p) {
   const int N = p.N, d = p.d;
   const int Np = ((N + 31) / 32) * 32;
+  sb_clear_steps(p.steps, p.B * p.H, N, p.K);
   const size_t e = (size_t)blockIdx.x * 256 + threadIdx.x;
   const size_t row = e / DP;
   const int c = (int)(e % DP);
@@ -227,7 +229,7 @@ __device__ __forceinline__ bf16x4 res_tr4(const bf16* op, int j0, int cb, int la
 }
 
 template <typename T, int DP, bool GEN, int OPS>
-__global__ void __launch_bounds__(UNR_NT) unrolled_bwd_kernel(UnrBwdArgs a) {
+__device__ __forceinline__ void unrolled_general(const UnrBwdArgs& a) {
   constexpr bool RES = OPS == UNR_OPS_RES;
   static_assert(!RES || (sizeof(T) == 2 && DP == 32), "resident operands: bf16, DP = 32");
   using M = Mfma<float, DP>;
@@ -954,6 +956,20 @@ __global__ void __launch_bounds__(UNR_NT) unrolled_bwd_kernel(UnrBwdArgs a) {
   }
 }
 
+template <typename T, int DP, bool GEN, int OPS>
+__global__ void __launch_bounds__(UNR_NT) unrolled_bwd_kernel(UnrBwdArgs a) {
+  unrolled_general<T, DP, GEN, OPS>(a);
+}
+// Register form (scaled_bwd.h); the general sweeps are a call, so that they cost its sweeps no registers.
+template <typename T, bool GEN>
+__device__ __attribute__((noinline)) void unrolled_general_call(UnrBwdArgs a) {
+  unrolled_general<T, 32, GEN, UNR_OPS_GLOBAL>(a);
+}
+template <typename T, bool GEN>
+__global__ void __launch_bounds__(SB_NT) unrolled_scaled_kernel(UnrBwdArgs a) {
+  scaled_bwd<T, GEN>(a, [](const UnrBwdArgs& x) { unrolled_general_call<T, GEN>(x); });
+}
+
 size_t unrolled_bwd_lds_bytes(int N, int DP, int elem, int ops) {
   const size_t Np = ((N + 31) / 32) * 32;
   size_t bytes = ((Np + 15) / 16) * 16;
@@ -993,9 +1009,8 @@ hipError_t launch_unrolled_prep(const UnrPrepArgs& p, bool bf16_in, int DP, hipS
   return hipErrorInvalidValue;
 }
 
-template <typename T, int DP, bool GEN, int OPS>
-static hipError_t launch_unr_t(const UnrBwdArgs& a, size_t lds, hipStream_t stream, bool coop) {
-  auto kern = unrolled_bwd_kernel<T, DP, GEN, OPS>;
+static hipError_t launch_unr_k(void (*kern)(UnrBwdArgs), const UnrBwdArgs& a, size_t lds, hipStream_t stream,
+                               bool coop) {
   hipError_t e = set_lds_limit((const void*)kern, lds);
   if (e != hipSuccess) return e;
   dim3 grid(grid_blocks(a.B * a.H, a.G)), block(UNR_NT);
@@ -1007,6 +1022,12 @@ static hipError_t launch_unr_t(const UnrBwdArgs& a, size_t lds, hipStream_t stre
   hipLaunchKernelGGL(kern, grid, block, lds, stream, copy);
   return hipGetLastError();
 }
+
+template <typename T, int DP, bool GEN, int OPS>
+static hipError_t launch_unr_t(const UnrBwdArgs& a, size_t lds, hipStream_t stream, bool coop) {
+  return launch_unr_k(unrolled_bwd_kernel<T, DP, GEN, OPS>, a, lds, stream, coop);
+}
+constexpr size_t UNR_STATIC = 4096;  // static LDS of the register form and the general sweeps, rounded up
 
 template <typename T>
 static hipError_t launch_unr_dt(const UnrBwdArgs& a, int DP, size_t lds, hipStream_t stream, bool coop, int ops) {
@@ -1025,8 +1046,19 @@ static hipError_t launch_unr_dt(const UnrBwdArgs& a, int DP, size_t lds, hipStre
 }
 
 // ops: from unrolled_operand_mode(), with lds sized for it
-hipError_t launch_unrolled_bwd(const UnrBwdArgs& a, bool bf16_in, int DP, size_t lds, hipStream_t stream, bool coop,
-                               int ops) {
+// The register form where the stripes and the iterations' vectors fit (limit: LDS of a workgroup).
+hipError_t launch_unrolled_bwd(const UnrBwdArgs& a, bool bf16_in, int DP, size_t lds, size_t limit, hipStream_t stream,
+                               bool coop, int ops) {
+  if (sb_fits(a.N, DP, a.G, a.K, false, limit - UNR_STATIC)) {
+    const bool gen = (a.bins8 && a.pos_w) || (a.has_geo && a.w_dist);
+    const size_t need = std::max(sb_lds_bytes(a.N, a.G, a.K, false),
+                                 unrolled_bwd_lds_bytes(a.N, DP, bf16_in ? 2 : 4, UNR_OPS_GLOBAL));
+    if (bf16_in)
+      return gen ? launch_unr_k(unrolled_scaled_kernel<bf16, true>, a, need, stream, coop)
+                 : launch_unr_k(unrolled_scaled_kernel<bf16, false>, a, need, stream, coop);
+    return gen ? launch_unr_k(unrolled_scaled_kernel<float, true>, a, need, stream, coop)
+               : launch_unr_k(unrolled_scaled_kernel<float, false>, a, need, stream, coop);
+  }
   return bf16_in ? launch_unr_dt<bf16>(a, DP, lds, stream, coop, ops)
                  : launch_unr_dt<float>(a, DP, lds, stream, coop, ops);
 }

@@ -115,7 +115,7 @@ class FlashSinkhornAttn(torch.autograd.Function):
         if mode == "unrolled":
             if int(K_iter) < 1:
                 raise ValueError("ift_mode='unrolled' needs K_iter >= 1")
-            hist = torch.zeros(int(K_iter), 2, B, H, N, **f32)
+            hist = torch.empty(int(K_iter), 2, B, H, N, **f32)
         lib = _lib.load()
         nbytes = lib.dfl_sinkhorn_workspace_size(B, H, N)
         ws = _lib.workspace(dev, nbytes)

@@ -63,7 +63,7 @@ def _run_forward(Q_s, K_s, x_res, V_h, eps, alpha_h, r_h, K_iter, mask):
     lu = torch.empty(B, H, N, **f32)
     lv = torch.empty(B, H, N, **f32)
     lz = torch.empty(B, H, N, **f32)
-    hist = torch.zeros(max(K_iter, 1), 2, B, H, N, **f32)
+    hist = torch.empty(max(K_iter, 1), 2, B, H, N, **f32)
     lib = _lib.load()
     ws = _lib.workspace(dev, lib.dfl_balanced_workspace_size(B, H, N, d, 0), "balanced")
     st = Qf.stride()

@@ -97,3 +97,69 @@ def test_register_balanced(B, H, N, d, K, eps, lengths):
     tol = 1e-4
     assert_close_rel(xc.cpu().double().numpy(), wx.numpy(), tol, "x_centroid")
     assert_close_rel(hc.cpu().double().numpy(), wh.numpy(), tol, "h_centroid")
+
+
+@pytest.mark.parametrize("B,H,N,d,K,eps,lengths,tol", [
+    (1, 8, 70, 32, 33, 1.0, None, 1e-4),          # odd iteration count, more than one batch of factors
+    (1, 4, 40, 16, 64, 1.0, None, 1e-4),          # the most iterations whose vectors are kept
+    (1, 4, 40, 16, 65, 1.0, None, 1e-4),          # one more: the general sweeps
+    (2, 8, 300, 32, 1, 0.5, [300, 163], 1e-4),    # a single iteration: no recurrence
+    (1, 8, 130, 32, 3, 0.03, [117], 1e-3),        # factors out of range: the general sweeps as a call
+])
+def test_register_balanced_gradients(B, H, N, d, K, eps, lengths, tol):
+    from deepfold_amd import balanced_sinkhorn_transport_dual
+
+    print(f"case B{B} H{H} N{N} d{d} K{K} eps{eps}", flush=True)
+    g = torch.Generator().manual_seed(N + K)
+    unit = lambda t: t / t.norm(dim=-1, keepdim=True)
+    leaves = dict(Q=unit(torch.randn(B, H, N, d, generator=g)), K=unit(torch.randn(B, H, N, d, generator=g)),
+                  x=3 * torch.randn(B, N, 3, generator=g), V=torch.randn(B, H, N, d, generator=g),
+                  al=-1 + 0.3 * torch.randn(H, generator=g), r=10 + torch.randn(H, generator=g))
+    e, mask = torch.full((H,), eps), None
+    if lengths is not None:
+        mask = torch.zeros(B, N)
+        for b, n in enumerate(lengths):
+            mask[b, :n] = 1
+    wx, wh = torch.randn(B, H, N, 3, generator=g), torch.randn(B, H, N, d, generator=g)
+    grads = []
+    for fn, conv in ((bt.balanced_transport_dual, lambda t: None if t is None else t.double()),
+                     (balanced_sinkhorn_transport_dual, lambda t: None if t is None else t.to(DEV))):
+        p = {k: conv(v).requires_grad_(True) for k, v in leaves.items()}
+        xc, hc = fn(p["Q"], p["K"], p["x"], p["V"], conv(e), p["al"], p["r"], K_iter=K, mask=conv(mask))
+        ((xc * conv(wx)).sum() + (hc * conv(wh)).sum()).backward()
+        grads.append({k: v.grad.detach().cpu().double().numpy() for k, v in p.items()})
+    for k in leaves:
+        assert_close_rel(grads[1][k], grads[0][k], tol, "d" + k)
+
+
+@pytest.mark.parametrize("B,H,N,d,K,lengths", [
+    (1, 4, 17, 32, 1, None),            # one iteration
+    (2, 8, 150, 32, 33, [150, 90]),     # odd count, several batches of factors; warm start
+    (1, 2, 40, 24, 65, None),           # past the kept iterations: the general sweeps
+])
+def test_register_unrolled_gradients(B, H, N, d, K, lengths):
+    from deepfold_amd import flash_sinkhorn_attn
+    from oracle import sinkhorn_dense_ref as dref
+
+    print(f"case B{B} H{H} N{N} d{d} K{K}", flush=True)
+    t = _uot(B, H, N, d, K, N + K, 0.3, lengths or [N] * B)
+    names = ("Q", "K", "V", "G", "log_mu", "log_nu")
+    go = torch.randn(B, N, H * d, generator=torch.Generator().manual_seed(3)) * t["mask"][:, :, None]
+    want = {k: np.zeros(t[k].shape) for k in names}
+    for b, n in enumerate(lengths or [N] * B):
+        p = {k: t[k][b:b + 1, :, :n].double().clone().requires_grad_(True) for k in names}
+        C = -(p["Q"] @ p["K"].transpose(-1, -2)) / math.sqrt(d)
+        lu, lv = dref.sinkhorn_solve(C, p["log_mu"], p["log_nu"], t["eps"].double(), K=K,
+                                     log_v_init=t["log_v_init"][b:b + 1, :, :n].double())
+        o, _, _ = dref.compute_transport_output(p["V"], p["G"], lu, lv, C, t["eps"].double())
+        (o * go[b:b + 1, :n].double()).sum().backward()
+        for k in names:
+            want[k][b:b + 1, :, :n] = p[k].grad.numpy()
+    c = {k: v.to(DEV) for k, v in t.items()}
+    p = {k: c[k].detach().requires_grad_(True) for k in names}
+    o = flash_sinkhorn_attn(p["Q"], p["K"], p["V"], p["G"], c["x_res"], c["pos_weight"], None, c["eps"], None,
+                            p["log_mu"], p["log_nu"], K_iter=K, log_v_init=c["log_v_init"], mask=c["mask"],
+                            ift_mode="unrolled")[0]
+    o.backward(go.to(DEV))
+    for k in names:
+        assert_close_rel(p[k].grad.cpu().double().numpy(), want[k], 1e-4, "d" + k)
