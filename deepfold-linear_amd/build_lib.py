@@ -17,7 +17,7 @@ OUT = os.path.join(HERE, "deepfold_amd", "libdfl_amd.so")
 OBJ_DIR = os.path.join(HERE, "_build")
 SOURCES = ["capi.hip", "sinkhorn_fwd.hip", "sinkhorn_fwd_stream.hip", "sinkhorn_fwd_reg.hip", "sinkhorn_fwd_reg_hist.hip",
            "sinkhorn_fwd_blk.hip", "sinkhorn_bwd.hip",
-           "sinkhorn_bwd_stream.hip", "attention.hip", "dense.hip", "balanced_bwd.hip",
+           "sinkhorn_bwd_stream.hip", "sinkhorn_bwd_reg.hip", "attention.hip", "dense.hip", "balanced_bwd.hip",
            "unrolled_bwd.hip", "trunk_steps.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # issue-rate / exchange probes (bench.py --workload peaks only): a library of its own

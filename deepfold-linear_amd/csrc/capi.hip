@@ -64,6 +64,10 @@ int balanced_max_tiles(int DP);
 hipError_t launch_balanced_prep(const BalPrepArgs& p, int DP, hipStream_t stream);
 hipError_t launch_balanced_bwd(const BalBwdArgs& a, int DP, size_t lds, size_t limit, hipStream_t stream, bool coop);
 size_t scaled_step_words(int N);
+bool sinkhorn_bwd_reg_n(int N, int G);
+bool sinkhorn_bwd_reg_fits(int N, int DP, int G, size_t lds_general, size_t limit);
+hipError_t launch_sinkhorn_bwd_reg(const IftBwdArgs& a, bool bf16_in, size_t lds_general, hipStream_t stream,
+                                   bool coop);
 hipError_t launch_balanced_finalize(const BalBwdArgs& a, float* dx, float* dalpha, float* dr, hipStream_t stream);
 size_t unrolled_bwd_lds_bytes(int N, int DP, int elem, int ops);
 int unrolled_operand_mode(int N, int DP, int elem, size_t limit);
@@ -294,11 +298,19 @@ constexpr int STREAM_VECS = 19;  // dfl::BWD_STREAM_VECS
 constexpr size_t LDS_LIMIT = 160 * 1024;
 // static LDS of the register-storage forward (its plan tables), beside the dynamic part
 constexpr size_t BLK_STATIC_LDS = 9 * 1024;
+// operands of the register-form backward: Q, K in rows and transposed, V and gO rows, gO
+// transposed, grad x_c and the coordinates
+size_t bwd_reg_bytes(int B, int H, int N, size_t elem) {
+  const size_t np = np32(N), bhn = (size_t)B * H * np;
+  return 4 * bhn * 32 * elem + 3 * bhn * 32 * 4 + bhn * 3 * 4 + (size_t)B * 3 * np * 4;
+}
 size_t stream_region_bytes(int B, int H, int N, int G) {
   const size_t np = np32(N);
   size_t b = 3 * prep_operand_bytes(B, H, N);
   b += ((size_t)B * np * 3 * 4 + 255) / 256 * 256;
   b += (size_t)B * H * G * STREAM_VECS * np * 4;
+  // the register-form backward keeps its operands here instead
+  if (dfl::sinkhorn_bwd_reg_n(N, G)) b = std::max(b, bwd_reg_bytes(B, H, N, 4));
   return (b + 255) / 256 * 256;
 }
 size_t stream_region_offset(int B, int H, int N, int G) {
@@ -842,6 +854,10 @@ int dfl_sinkhorn_bwd(const dfl_sinkhorn_bwd_params* p, void* workspace, size_t w
   if (int rc = acquire_salt(ws, WS_HEADER + xch_words(p->B, p->H, p->N) * 8, stream, &a.salt))
     return hip_fail((hipError_t)rc, "workspace clear launch");
   a.ch = CH;
+  // the plan in registers where the stripes fit the register tiles (its operands take the stream
+  // region, unused there)
+  const bool reg_mode = !stream_mode && p->storage == DFL_STORAGE_AUTO &&
+                        dfl::sinkhorn_bwd_reg_fits(p->N, DP, G, lds, LDS_LIMIT);
   if (p->pos_bins)
     if (int rc = prepare_bins8(p->pos_bins, p->B, p->N, workspace, sinkhorn_bins8_offset(p->B, p->H, p->N),
                                &a.bins8, &a.bins8t, stream))
@@ -849,7 +865,7 @@ int dfl_sinkhorn_bwd(const dfl_sinkhorn_bwd_params* p, void* workspace, size_t w
   // a workspace with room for the bias matrices: the per-element bins lookups and
   // distances are evaluated once here instead of in every sweep
   const bool has_bias = (p->pos_bins && p->pos_weight) || (p->x_res && p->w_dist);
-  if (has_bias && workspace_bytes >= need + dfl_sinkhorn_bias_workspace_size(p->B, p->H, p->N)) {
+  if (!reg_mode && has_bias && workspace_bytes >= need + dfl_sinkhorn_bias_workspace_size(p->B, p->H, p->N)) {
     float* mat = reinterpret_cast<float*>(ws + bias_mat_offset(p->B, p->H, p->N));
     float* matT = mat + (size_t)p->B * p->H * np32(p->N) * np32(p->N);
     hipError_t e = dfl::launch_bias_mat(a, mat, matT, (hipStream_t)stream);
@@ -858,6 +874,38 @@ int dfl_sinkhorn_bwd(const dfl_sinkhorn_bwd_params* p, void* workspace, size_t w
     a.bias_matT = matT;
   }
   const bool coop = coop_launch(G, a.B * a.H);
+  if (reg_mode) {
+    const size_t bhn = (size_t)p->B * p->H * np32(p->N);
+    unsigned char* at = ws + stream_region_offset(p->B, p->H, p->N, G);
+    auto carve = [&](size_t bytes) { unsigned char* q = at; at += bytes; return q; };
+    dfl::UnrPrepArgs pr;
+    memset(&pr, 0, sizeof(pr));
+    pr.q = p->q; pr.k = p->k; pr.v = p->v; pr.g = p->g;
+    pr.sb = p->stride_b; pr.sh = p->stride_h; pr.sn = p->stride_n;
+    pr.x = p->x_res; pr.mask = p->mask; pr.o_avg = p->o_avg; pr.xc = p->x_centroid;
+    pr.grad_o = p->grad_o; pr.grad_xc = p->grad_xc;
+    pr.B = p->B; pr.H = p->H; pr.N = p->N; pr.d = p->d;
+    const size_t opb = bhn * 32 * elem, fpb = bhn * 32 * 4;  // multiples of 16 bytes: np is one of 32
+    pr.qp = carve(opb); pr.kp = carve(opb); pr.qt = carve(opb); pr.kt = carve(opb);
+    pr.vp = reinterpret_cast<float*>(carve(fpb)); pr.gp = reinterpret_cast<float*>(carve(fpb));
+    pr.gt = reinterpret_cast<float*>(carve(fpb)); pr.gxs = reinterpret_cast<float*>(carve(bhn * 3 * 4));
+    pr.xs = reinterpret_cast<float*>(carve((size_t)p->B * 3 * np32(p->N) * 4));
+    pr.dcoef = a.dcoef; pr.dg = p->dg;
+    pr.go_hi = a.go_hi; pr.go_lo = a.go_lo; pr.go_t = a.go_t;
+    hipError_t e = dfl::launch_unrolled_prep(pr, p->dtype == DFL_BF16, DP, (hipStream_t)stream);
+    if (e != hipSuccess) return hip_fail(e, "sinkhorn backward prep launch");
+    dfl::IftBwdArgs ia;
+    static_cast<dfl::SinkBwdArgs&>(ia) = a;
+    ia.qp = pr.qp; ia.kp = pr.kp; ia.qt = pr.qt; ia.kt = pr.kt; ia.vp = pr.vp; ia.gp = pr.gp; ia.gt = pr.gt;
+    ia.gxs = pr.gxs; ia.xs = pr.xs;
+    e = dfl::launch_sinkhorn_bwd_reg(ia, p->dtype == DFL_BF16, lds, (hipStream_t)stream, coop);
+    if (e != hipSuccess) return hip_fail(e, "sinkhorn backward launch");
+    if (p->dx_res || p->dpos_weight || p->dw_dist) {
+      e = dfl::launch_sinkhorn_bwd_finalize(a, p->dx_res, p->dpos_weight, p->dw_dist, (hipStream_t)stream);
+      if (e != hipSuccess) return hip_fail(e, "sinkhorn backward finalize launch");
+    }
+    return 0;
+  }
   hipError_t e = dfl::launch_sinkhorn_bwd_prep(a, p->dtype == DFL_BF16, DP, (hipStream_t)stream);
   if (e != hipSuccess) return hip_fail(e, "sinkhorn backward prep launch");
   if (stream_mode) {

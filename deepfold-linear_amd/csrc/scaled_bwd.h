@@ -1,4 +1,5 @@
-// Unrolled backwards (balanced transport and UOT flash-Sinkhorn) with the plan in registers.
+// Backwards with the plan in registers: unrolled (balanced transport and UOT flash-Sinkhorn) and
+// implicit (UOT).
 //
 // The plans of all half-iterations share one matrix: with E_ij = exp(L_ij + alpha_i + beta_j)
 // and the last iteration's potentials as alpha, beta (E = P, rows summing to 1),
@@ -17,11 +18,16 @@
 // follow in that one pass.  The sweeps that recompute the cost and form both terms of every
 // iteration (balanced_bwd.hip, unrolled_bwd.hip) took 7-8 us each; these take about 1.5-2 us.
 //
+// The implicit (IFT) backward is the same with one pair of factors: S_row = E, S_col = E AC BC with
+// AC_i = exp(log Z_i), BC_j = exp(-(v_j + col_lse_j)), R_ij = -z_u,i -+ AC_i BC_j z_v,j, and its solve
+// (fixed point, or CG on W = AC^1/2 E BC^1/2) takes one multiply-add per element and sweep.
+//
 // A wave keeps E of its pairs in both orientations, as the register forward (reg_ks, reg_nrm).
 // Every factor must lie within 2^+-SB_MAX: E <= 1, so an entry that underflows (below 2^-126)
 // then stays below 2^-62 in every plan.  The members of a group agree on that from the recorded
 // potentials before they begin; a group outside it runs the general sweeps.
 #pragma once
+#include "sinkhorn_bwd_kernel.h"
 #include "sinkhorn_fwd_kernel.h"
 
 namespace dfl {
@@ -46,6 +52,9 @@ __device__ __forceinline__ void sb_clear_steps(uint64_t* steps, int BH, int N, i
 }
 
 template <typename Args> struct is_bal : std::is_same<Args, BalBwdArgs> {};
+template <typename Args> struct is_ift : std::is_same<Args, IftBwdArgs> {};
+
+constexpr int SB_BINS = (BIN_NONE + 4) / 4 * 4;  // (the tables are followed by 16-byte reads)
 
 // floats of the region that holds the stripe's factors and vectors (AC, BR, y, z and, UOT, AR, BC)
 // during the sweeps and the waves' output partials afterwards
@@ -56,7 +65,13 @@ __host__ __device__ inline int sb_region_floats(int N, int G, int K, bool bal) {
 }
 inline size_t sb_lds_bytes(int N, int G, int K, bool bal) {
   const size_t Np = ((N + 31) / 32) * 32, cpn = reg_cp_rows(N, (int)Np);
-  return ((Np + 15) / 16) * 16 + (7 * Np + 2 * cpn + 2 * (size_t)SB_NW * SK_RT * 16 + sb_region_floats(N, G, K, bal)) * 4;
+  return ((Np + 15) / 16) * 16 + (7 * Np + 2 * cpn + 2 * SB_BINS + 2 * (size_t)SB_NW * SK_RT * 16 + sb_region_floats(N, G, K, bal)) * 4;
+}
+// IFT: the CG vectors (5 Np) and three vectors of the stripe take the factors' place
+inline size_t ift_lds_bytes(int N, int G) {
+  const size_t Np = ((N + 31) / 32) * 32, cpn = reg_cp_rows(N, (int)Np), loc = fwd_local_rows(N, G);
+  const size_t f = 5 * Np + 3 * loc, m = (loc / 16) * SB_NW * 8 * WAVE;
+  return ((Np + 15) / 16) * 16 + (7 * Np + 2 * cpn + 2 * SB_BINS + 2 * (size_t)SB_NW * SK_RT * 16 + (f > m ? f : m)) * 4;
 }
 inline bool sb_fits(int N, int DP, int G, int K, bool bal, size_t limit) {
   return DP == 32 && K >= 1 && K <= SB_KMAX && reg_fits(N, G) && sb_lds_bytes(N, G, K, bal) + 2048 <= limit;
@@ -66,17 +81,19 @@ inline bool sb_fits(int N, int DP, int G, int K, bool bal, size_t limit) {
 // the balanced mode); general(a): the general sweeps, for a group whose factors are out of range.
 template <typename T, bool GEN, typename Args, typename General>
 __device__ __forceinline__ void scaled_bwd(const Args& a, General general) {
-  constexpr bool BAL = is_bal<Args>::value;
+  constexpr bool BAL = is_bal<Args>::value, IFT = is_ift<Args>::value, UNR = !BAL && !IFT;
   constexpr int DP = 32, NC = DP / 16;
   using MQ = Mfma<T, DP>;
   using M = Mfma<float, DP>;
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ int s_flagp[2], s_tmp, s_flag, s_local, s_ok, s_cnt;
-  __shared__ float s_pw[BIN_NONE + 1], s_posw[BIN_NONE + 1], s_dpw[BIN_NONE + 1], sscal[2 * SB_NW];
+  __shared__ float sscal[2 * SB_NW], s_red[2 * SB_NW];
   int grp, member;
   if (!group_of(a.B * a.H, a.G, grp, member)) return;
   const int b = grp / a.H, h = grp % a.H;
-  const int N = a.N, d = a.d, K = a.K, BH = a.B * a.H;
+  const int N = a.N, d = a.d, BH = a.B * a.H;
+  int K = 0;  // (IFT: no recorded iterations)
+  if constexpr (!IFT) K = a.K;
   const int Np = ((N + 31) / 32) * 32;
   const size_t bh = (size_t)grp, bhN = bh * N;
   const int tid = threadIdx.x, lane = tid & (WAVE - 1), g = lane >> 4;
@@ -93,7 +110,9 @@ __device__ __forceinline__ void scaled_bwd(const Args& a, General general) {
   const int cpn = reg_cp_rows(N, Np), loc = fwd_local_rows(N, a.G);
   float* wY = dcf + Np;   // beta (log2), then y^k of this wave's streamed columns
   float* wZ = wY + cpn;   // alpha (log2), then z^k of this wave's streamed rows
-  float* scratch = wZ + cpn;                       // two slots of wave partials
+  float* s_posw = wZ + cpn;                        // bin weights in the exponent, and their gradients
+  float* s_dpw = s_posw + SB_BINS;
+  float* scratch = s_dpw + SB_BINS;                // two slots of wave partials
   float* region = scratch + 2 * SB_NW * SK_RT * 16;
   float* AC = region;                              // [K][loc] each
   float* BR = AC + (size_t)K * loc;
@@ -101,6 +120,15 @@ __device__ __forceinline__ void scaled_bwd(const Args& a, General general) {
   float* Zo = Yo + (size_t)K * loc;
   float* AR = BAL ? AC : Zo + (size_t)K * loc;
   float* BC = BAL ? nullptr : AR + (size_t)K * loc;
+  // IFT: CG vectors [Np] each (region), then z_u, BC z_v and AC of my rows / columns
+  float* cy = region;
+  float* cr = cy + Np;
+  float* cp = cr + Np;
+  float* cs = cp + Np;
+  float* bch = cs + Np;
+  float* zo = bch + Np;
+  float* yo = zo + loc;
+  float* ao = yo + loc;
 
   const int n = mask_setup(a.mask ? a.mask + (size_t)b * N : nullptr, N, valid, &s_tmp);
   const int n_tiles = (n + 15) / 16;
@@ -122,13 +150,13 @@ __device__ __forceinline__ void scaled_bwd(const Args& a, General general) {
     kappa = a.lam / (a.lam + eps);
     wd = a.w_dist ? a.w_dist[h] : 0.f;
     if (tid <= (int)BIN_NONE) {
-      s_pw[tid] = a.pos_w && tid < (int)BIN_NONE ? a.pos_w[h * 68 + tid] : 0.f;
-      s_posw[tid] = -LOG2E * s_pw[tid] / eps;
+      s_posw[tid] = a.pos_w && tid < (int)BIN_NONE ? -LOG2E * a.pos_w[h * 68 + tid] / eps : 0.f;
       s_dpw[tid] = 0.f;
     }
   }
   const float ik = 1.f / kappa;
-  const float* hist = a.hist;
+  const float* hist = nullptr;
+  if constexpr (!IFT) hist = a.hist;
   auto Uat = [&](int k) { return hist + ((size_t)(2 * k + 1) * BH + bh) * N; };
   auto Vat = [&](int k) { return hist + ((size_t)(2 * k) * BH + bh) * N; };
   // natural units; alpha without the balanced beta's -lm
@@ -136,10 +164,13 @@ __device__ __forceinline__ void scaled_bwd(const Args& a, General general) {
     if constexpr (BAL) return Uat(K - 1)[i];
     else return a.log_u[bhN + i] - a.log_z[bhN + i];
   };
-  auto beta_of = [&](int j) -> float { return Vat(K - 1)[j]; };
+  auto beta_of = [&](int j) -> float {
+    if constexpr (IFT) return a.log_v[bhN + j];
+    else return Vat(K - 1)[j];
+  };
   auto vprev = [&](int k, int j) -> float {  // v^{k-1}
     if (k >= 1) return Vat(k - 1)[j];
-    if constexpr (BAL) return 0.f;
+    if constexpr (!UNR) return 0.f;
     else return a.v_init ? a.v_init[bhN + j] : 0.f;
   };
   auto urow = [&](int k, int i) -> float {  // the row potential of AC_k
@@ -158,7 +189,7 @@ __device__ __forceinline__ void scaled_bwd(const Args& a, General general) {
         if (!BAL || k >= 1) in = in && fabsf(eb) <= SB_MAX;
         ac = fast_exp2(ea);
         br = BAL && k == 0 ? 0.f : fast_exp2(eb);
-        if constexpr (!BAL) {
+        if constexpr (UNR) {
           const float er = (u * ik - a.log_mu[bhN + i] - al) * LOG2E;
           const float ec = (Vat(k)[i] * ik - a.log_nu[bhN + i] - be) * LOG2E;
           in = in && fabsf(er) <= SB_MAX && fabsf(ec) <= SB_MAX;
@@ -169,16 +200,31 @@ __device__ __forceinline__ void scaled_bwd(const Args& a, General general) {
       AC[(size_t)k * loc + q] = ac;
       BR[(size_t)k * loc + q] = br;
       Yo[(size_t)k * loc + q] = Zo[(size_t)k * loc + q] = 0.f;
-      if constexpr (!BAL) {
+      if constexpr (UNR) {
         AR[(size_t)k * loc + q] = ar;
         BC[(size_t)k * loc + q] = bc;
+      }
+    }
+    if constexpr (IFT) {
+      for (int q = tid; q < nr * 16; q += SB_NT) {
+        const int i = r_lo + q;
+        if (i < n && valid[i])
+          in = in && fabsf(a.log_z[bhN + i] * LOG2E) <= SB_MAX &&
+               fabsf((a.log_v[bhN + i] + a.col_lse[bhN + i]) * LOG2E) <= SB_MAX;
       }
     }
     if (!in) s_ok = 0;  // (the same value from every writer)
   }
   __syncthreads();
-  uint64_t* steps = a.steps + bh * sb_step_words(N);
-  uint64_t* verdicts = steps + (size_t)2 * SB_KMAX * Np;
+  uint64_t* steps;
+  uint64_t* verdicts;
+  if constexpr (IFT) {
+    steps = a.xch + bh * 4 * (size_t)Np;  // three vectors reused by every iteration; the fourth is free
+    verdicts = steps + 3 * (size_t)Np;
+  } else {
+    steps = a.steps + bh * sb_step_words(N);
+    verdicts = steps + (size_t)2 * SB_KMAX * Np;
+  }
   const uint32_t salt = a.salt << 12;
   if (tid == 0) xch_put(verdicts + member, (s_ok ? 0.f : 2.f) + (xcc_placed() ? 0.f : 1.f), salt | 1u);
   for (int i = tid; i < Np; i += SB_NT) {
@@ -218,10 +264,9 @@ __device__ __forceinline__ void scaled_bwd(const Args& a, General general) {
     }
     if (tid < 3) a.dx_part[(bhN + i) * 3 + tid] = 0.f;
     if constexpr (!BAL)
-      if (tid == 0) {
-        a.dlog_mu[bhN + i] = a.dlog_nu[bhN + i] = 0.f;
-        if (a.dv_init) a.dv_init[bhN + i] = 0.f;
-      }
+      if (tid == 0) a.dlog_mu[bhN + i] = a.dlog_nu[bhN + i] = 0.f;
+    if constexpr (UNR)
+      if (tid == 0 && a.dv_init) a.dv_init[bhN + i] = 0.f;
   }
   float sc, r0;
   bool geo, use_bins = false, has_h = true;
@@ -237,8 +282,10 @@ __device__ __forceinline__ void scaled_bwd(const Args& a, General general) {
     sc = LOG2E / (sqrtf((float)d) * eps);
     r0 = a.r0;
     bias.geo_scale = -LOG2E * wd / eps;
-    geo = GEN && a.has_geo != 0 && wd != 0.f;
-    use_bins = GEN && a.bins8 != nullptr;
+    // (IFT: d w_dist is non-zero even where w_dist == 0)
+    if constexpr (IFT) geo = GEN && a.x != nullptr && a.w_dist != nullptr;
+    else geo = GEN && a.has_geo != 0 && wd != 0.f;
+    use_bins = GEN && a.bins8 != nullptr && a.pos_w != nullptr;
     if (use_bins) {
       bias.b8 = a.bins8 + (size_t)b * Np * Np;
       bias.b8t = a.bins8t + (size_t)b * Np * Np;
@@ -366,8 +413,161 @@ __device__ __forceinline__ void scaled_bwd(const Args& a, General general) {
     // combining thread of local row / column qc
     const int qc = tid, ic = r_lo + qc;
     const bool has_q = qc < nr * 16, in_c = has_q && ic < n, ok_c = in_c && valid[ic];
-    float dmu = 0.f, dnu = 0.f, dv0 = 0.f;
+    constexpr int NB = (16 * KSL + WAVE - 1) / WAVE;  // words of a lane
     auto words_of = [&](int k, int z) { return steps + (size_t)(2 * k + z) * Np; };
+    if constexpr (IFT) {
+      uint64_t* xG = steps;
+      uint64_t* xZ = steps + Np;
+      uint64_t* xY = steps + 2 * (size_t)Np;
+      const float lz_c = ok_c ? a.log_z[bhN + ic] * LOG2E : 0.f;
+      const float vc_c = ok_c ? (a.log_v[bhN + ic] + a.col_lse[bhN + ic]) * LOG2E : 0.f;
+      const float ac_c = ok_c ? fast_exp2(lz_c) : 0.f, bc_c = ok_c ? fast_exp2(-vc_c) : 0.f;
+      const float gv_c = has_q ? reg_sum<SB_NW>(scratch, qc) : 0.f;
+      float zu_c = 0.f, zv_c = gv_c;
+      auto take0 = [&](float* w) {
+        return [w](int, int i, float v, bool ok) {
+          w[i] = ok ? v : 0.f;
+          return 0.f;
+        };
+      };
+      float dm;
+      if (a.solver == 0) {
+        // Gauss-Seidel (flash_sinkhorn_attn.py:471-542) from z_v = g_v: z_u = kappa S_col z_v,
+        // z_v = g_v + kappa S_row^T z_u, with y = BC z_v exchanged
+        ++phase;
+        if (in_c) xch_put(xY + ic, bc_c * zv_c, salt | phase, local);
+        for (int it = 0; it < a.iters; ++it) {
+          if (!wave_poll<SB_NW, NB>(xY, n, n_tiles, salt | phase, valid, a.err, dm, take0(wY))) s_flagp[phase & 1] = 1;
+          float* part = part_slot();
+          reg_scaled<KSL, NRM, SB_NW>(XR, nr, wY, part);
+          ++phase;
+          lds_barrier();
+          if (has_q) {
+            zu_c = kappa * ac_c * reg_sum<SB_NW>(part, qc);
+            if (in_c) xch_put(xZ + ic, zu_c, salt | phase, local);
+          }
+          lds_barrier();
+          if (s_flagp[(phase - 1) & 1]) return;
+          if (!wave_poll<SB_NW, NB>(xZ, n, n_tiles, salt | phase, valid, a.err, dm, take0(wZ))) s_flagp[phase & 1] = 1;
+          part = part_slot();
+          reg_scaled<KSL, NRM, SB_NW>(XC, nr, wZ, part);
+          ++phase;
+          lds_barrier();
+          if (has_q) {
+            zv_c = gv_c + kappa * reg_sum<SB_NW>(part, qc);
+            if (in_c) xch_put(xY + ic, bc_c * zv_c, salt | phase, local);
+          }
+          lds_barrier();
+          if (s_flagp[(phase - 1) & 1]) return;
+        }
+        if (!wave_poll<SB_NW, NB>(xY, n, n_tiles, salt | phase, valid, a.err, dm, take0(wY))) s_flagp[phase & 1] = 1;
+        if (a.iters == 0)
+          for (int e = lane; e < 16 * KSL; e += WAVE) wZ[min((wave + SB_NW * (e >> 4)) * 16 + (e & 15), cpn - 1)] = 0.f;
+        __syncthreads();
+        if (s_flagp[phase & 1]) return;
+      } else {
+        // CG on (I - kappa^2 W^T W) y = BC^1/2 g_v, W = AC^1/2 E BC^1/2; the vectors are kept whole and
+        // bit-identical in every member, as in the general backward.  t travels as AC^1/2 t.
+        ++phase;
+        if (in_c) xch_put(xG + ic, gv_c, salt | phase, local);
+        if (!gather_vector(xG, n, Np, salt | phase, cr, valid, a.err, &s_flag)) return;
+        for (int i = tid; i < Np; i += SB_NT) {
+          const bool ok = i < n && valid[i];
+          const float h_ = ok ? fast_exp2(-0.5f * (a.log_v[bhN + i] + a.col_lse[bhN + i]) * LOG2E) : 0.f;
+          const float bj = cr[i] * h_;
+          bch[i] = h_;
+          cy[i] = 0.f;
+          cr[i] = bj;
+          cp[i] = bj;
+        }
+        __syncthreads();
+        int flip = 0;
+        float rr = block_sum(Np, [&](int i) { return cr[i] * cr[i]; }, s_red, flip);
+        const bool early_exit = a.cg_rtol > 0.f;
+        const float stop2 = a.cg_rtol * a.cg_rtol * rr, k2 = kappa * kappa;
+        const float ach_c = ok_c ? fast_exp2(0.5f * lz_c) : 0.f, bch_c = ok_c ? fast_exp2(-0.5f * vc_c) : 0.f;
+        float zs[NB], tt[NB], zsum_c = 0.f;
+#pragma unroll
+        for (int s_ = 0; s_ < NB; ++s_) zs[s_] = tt[s_] = 0.f;
+        for (int it = 0; it < a.iters; ++it) {
+          if (early_exit && (rr <= stop2 || rr == 0.f)) break;
+          // the wave's own streamed columns of BC^1/2 p (it updated them itself)
+#pragma unroll
+          for (int s_ = 0; s_ < NB; ++s_) {
+            const int e = s_ * WAVE + lane, i = (wave + SB_NW * (e >> 4)) * 16 + (e & 15);
+            if (e < 16 * KSL && i < n_tiles * 16) wY[i] = bch[i] * cp[i];
+          }
+          float* part = part_slot();
+          reg_scaled<KSL, NRM, SB_NW>(XR, nr, wY, part);
+          ++phase;
+          lds_barrier();
+          float tt_c = 0.f;
+          if (has_q) {
+            tt_c = ach_c * (ach_c * reg_sum<SB_NW>(part, qc));
+            if (in_c) xch_put(xZ + ic, tt_c, salt | phase, local);
+          }
+          if (!wave_poll<SB_NW, NB>(xZ, n, n_tiles, salt | phase, valid, a.err, dm, [&](int s_, int i, float v, bool ok) {
+                wZ[i] = ok ? v : 0.f;
+#pragma unroll
+                for (int u = 0; u < NB; ++u)
+                  if (u == s_) tt[u] = ok ? v : 0.f;
+                return 0.f;
+              }))
+            s_flag = 1;
+          part = part_slot();
+          reg_scaled<KSL, NRM, SB_NW>(XC, nr, wZ, part);
+          ++phase;
+          lds_barrier();
+          if (has_q && in_c) xch_put(xY + ic, bch_c * reg_sum<SB_NW>(part, qc), salt | phase, local);
+          float pAp;
+          if (!gather_vector_dot(xY, n, Np, salt | phase, cs, valid, a.err, &s_flag,
+                                 [&](int i) { return cp[i] * (cp[i] - k2 * cs[i]); }, s_red, flip, &pAp))
+            return;
+          if (early_exit && pAp == 0.f) break;
+          const float alpha = (pAp != 0.f && rr != 0.f) ? rr / pAp : 0.f;
+          const float rr_new = block_sum(Np, [&](int i) {
+            cy[i] += alpha * cp[i];
+            const float ri = cr[i] - alpha * (cp[i] - k2 * cs[i]);
+            cr[i] = ri;
+            return ri * ri;
+          }, s_red, flip);
+          zsum_c += alpha * tt_c;
+#pragma unroll
+          for (int s_ = 0; s_ < NB; ++s_) zs[s_] += alpha * tt[s_];
+          const float beta = rr != 0.f ? rr_new / rr : 0.f;
+          rr = rr_new;
+          // each wave updates p where its own next row sweep reads it: no barrier
+#pragma unroll
+          for (int s_ = 0; s_ < NB; ++s_) {
+            const int e = s_ * WAVE + lane, i = (wave + SB_NW * (e >> 4)) * 16 + (e & 15);
+            if (e < 16 * KSL && i < n_tiles * 16) cp[i] = cr[i] + beta * cp[i];
+          }
+        }
+        zu_c = kappa * zsum_c;
+        zv_c = ok_c ? cy[ic] * fast_exp2(0.5f * vc_c) : 0.f;
+#pragma unroll
+        for (int s_ = 0; s_ < NB; ++s_) {
+          const int e = s_ * WAVE + lane, i = (wave + SB_NW * (e >> 4)) * 16 + (e & 15);
+          if (e < 16 * KSL && i < n_tiles * 16) {
+            wY[i] = bch[i] * cy[i];
+            wZ[i] = kappa * zs[s_];
+          }
+        }
+      }
+      if (has_q) {
+        zo[qc] = ok_c ? zu_c : 0.f;
+        yo[qc] = bc_c * zv_c;
+        ao[qc] = ac_c;
+        if (ic < N) {
+          // analytic: d log_mu = kappa lambda_u = -kappa z_u
+          a.dlog_mu[bhN + ic] = ok_c ? (a.mode == 1 ? -kappa : kappa) * zu_c : 0.f;
+          a.dlog_nu[bhN + ic] = ok_c ? kappa * zv_c : 0.f;
+        }
+      }
+      __syncthreads();
+    }
+    if constexpr (!IFT) {
+    float dmu = 0.f, dnu = 0.f, dv0 = 0.f;
     auto publish_y = [&](int k, float hv) {  // h^k of my column -> y^k
       const float y = BAL ? (k == K - 1 ? hv : BR[(size_t)(k + 1) * loc + qc] * hv) : BC[(size_t)k * loc + qc] * hv;
       Yo[(size_t)k * loc + qc] = ok_c ? y : 0.f;
@@ -387,7 +587,7 @@ __device__ __forceinline__ void scaled_bwd(const Args& a, General general) {
     for (int k = K - 1; k >= K_END; --k) {
       {  // row half: g^k, z^k
         float dm;
-        if (!wave_poll<SB_NW, (16 * KSL + WAVE - 1) / WAVE>(words_of(k, 0), n, n_tiles, salt | phase, valid, a.err, dm, take(wY)))
+        if (!wave_poll<SB_NW, NB>(words_of(k, 0), n, n_tiles, salt | phase, valid, a.err, dm, take(wY)))
           s_flagp[phase & 1] = 1;
         float* part = part_slot();
         reg_scaled<KSL, NRM, SB_NW>(XR, nr, wY, part);
@@ -405,7 +605,7 @@ __device__ __forceinline__ void scaled_bwd(const Args& a, General general) {
       }
       {  // column half: h^{k-1}, y^{k-1}
         float dm;
-        if (!wave_poll<SB_NW, (16 * KSL + WAVE - 1) / WAVE>(words_of(k, 1), n, n_tiles, salt | phase, valid, a.err, dm, take(wZ)))
+        if (!wave_poll<SB_NW, NB>(words_of(k, 1), n, n_tiles, salt | phase, valid, a.err, dm, take(wZ)))
           s_flagp[phase & 1] = 1;
         float* part = part_slot();
         reg_scaled<KSL, NRM, SB_NW>(XC, nr, wZ, part);
@@ -422,12 +622,12 @@ __device__ __forceinline__ void scaled_bwd(const Args& a, General general) {
     }
     if constexpr (BAL) {  // y^0 has no row half: the last pass reads its words
       float dm;
-      if (!wave_poll<SB_NW, (16 * KSL + WAVE - 1) / WAVE>(words_of(0, 0), n, n_tiles, salt | phase, valid, a.err, dm, take(wY)))
+      if (!wave_poll<SB_NW, NB>(words_of(0, 0), n, n_tiles, salt | phase, valid, a.err, dm, take(wY)))
         s_flagp[phase & 1] = 1;
       __syncthreads();
       if (s_flagp[phase & 1]) return;
     }
-    if constexpr (!BAL) {
+    if constexpr (UNR) {
       if (in_c) {
         a.dlog_mu[bhN + ic] = ok_c ? dmu : 0.f;
         a.dlog_nu[bhN + ic] = ok_c ? dnu : 0.f;
@@ -438,6 +638,7 @@ __device__ __forceinline__ void scaled_bwd(const Args& a, General general) {
       }
     }
     __syncthreads();
+    }
 
     // ---- the cost gradient and everything that follows from it, one pass per orientation
     float gb[NRM][3], xt[NRM][3], s_al = 0.f, s_r = 0.f, s_w = 0.f;
@@ -469,7 +670,8 @@ __device__ __forceinline__ void scaled_bwd(const Args& a, General general) {
           for (int r = 0; r < NRM; ++r) R[r] = f32x4{0.f, 0.f, 0.f, 0.f};
           const int si = st * 16 + (lane & 15);
           const bool sok = si < n && valid[si];
-          const float sbase = sok ? (ROW ? beta_of(si) : alpha_of(si)) : 0.f;
+          float sbase = 0.f;
+          if constexpr (!IFT) sbase = sok ? (ROW ? beta_of(si) : alpha_of(si)) : 0.f;
           // the tile's operands, in flight with the first batch of factors
           typename M::Frag cf;
           typename MQ::Frag fs;
@@ -483,6 +685,7 @@ __device__ __forceinline__ void scaled_bwd(const Args& a, General general) {
             op[c] = *reinterpret_cast<const reg_vt<T>*>((ROW ? kt : qt) + o);
             if (!ROW && has_h) go[c] = *reinterpret_cast<const f32x4*>(gt + o);
           }
+          if constexpr (!IFT) {
           // this lane's streamed factor of iteration kk = 2 s + (g >> 1), one pointer step a slot
           const float* p = from_words ? reinterpret_cast<const float*>(words_of(g >> 1, ROW ? 0 : 1) + si) + 1
                                       : hist + ((long long)(2 * ((g >> 1) - (shifted ? 1 : 0)) + (ROW ? 0 : 1)) * BH + (long long)bh) * N + si;
@@ -515,6 +718,27 @@ __device__ __forceinline__ void scaled_bwd(const Args& a, General general) {
               bp += 2 * loc;
               kb += 2;
             }
+          }
+          } else {
+            // R_ij = -z_u,i + sgn AC_i y_j (sgn -1, analytic +1)
+            const float sgn = a.mode == 1 ? 1.f : -1.f;
+            const f32x4 wv = *reinterpret_cast<const f32x4*>((ROW ? wY : wZ) + st * 16 + 4 * g);
+            f32x4 as = {0.f, 0.f, 0.f, 0.f};
+            if (!ROW) {
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                const int i = st * 16 + 4 * g + e;
+                if (i < n && valid[i]) as[e] = sgn * fast_exp2(a.log_z[bhN + i] * LOG2E);
+              }
+            }
+#pragma unroll
+            for (int r = 0; r < NRM; ++r)
+              if (r < nr) {
+                const int q = r * 16 + (lane & 15);
+                const float m = ROW ? sgn * ao[q] : yo[q], z0 = ROW ? zo[q] : 0.f;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) R[r][e] = ROW ? __builtin_fmaf(m, wv[e], -z0) : __builtin_fmaf(as[e], m, -wv[e]);
+              }
           }
           float xv[12], gv[12];
           vec3(xs + 3 * (st * 16 + 4 * g), xv);

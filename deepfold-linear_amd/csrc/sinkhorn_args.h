@@ -198,6 +198,18 @@ struct UnrBwdArgs {
   uint32_t salt;
 };
 
+// IFT backward in register form: the general one's arguments and the prepared operands of the
+// unrolled backward's prep kernel (UnrPrepArgs).
+struct IftBwdArgs : SinkBwdArgs {
+  const void* qt;        // [B*H][DP][Np] in the input type (qp, kp: SinkBwdArgs)
+  const void* kt;
+  const float* vp;       // V rows
+  const float* gp;       // gO rows
+  const float* gt;       // gO transposed
+  const float* gxs;      // [B*H][3][Np] grad x_c
+  const float* xs;       // [B][3][Np] coordinates
+};
+
 struct UnrPrepArgs {
   const void* q;  // (B,H,N,d) bf16 or fp32, element strides sb/sh/sn
   const void* k;
@@ -216,8 +228,9 @@ struct UnrPrepArgs {
   float* vp; float* gp; float* gt;
   float* dcoef; float* gxs; float* xs;
   void* dg;              // (B,H,N,d) in the input type, or null (no gate)
-  uint64_t* steps;       // kept exchange words of the register form, cleared for K iterations
+  uint64_t* steps;       // kept exchange words of the register form, cleared for K iterations (or null)
   int K;
+  void* go_hi; void* go_lo; void* go_t;  // the general IFT backward's gO operands (SinkBwdArgs), or null
 };
 
 struct BalPrepArgs {

@@ -690,7 +690,7 @@ __host__ __device__ inline int bwd_local_rows(int N, int G) { return 16 * (((N +
 // GEN: the cost may carry position bins or geometry (set by the host when either is
 // passed); GEN = false compiles no bias code.
 template <typename T, int DP, bool STREAM, bool GEN>
-__global__ void __launch_bounds__(BWD_NT) sinkhorn_bwd_kernel(SinkBwdArgs a) {
+__device__ __forceinline__ void sinkhorn_bwd_general(const SinkBwdArgs& a) {
   using M = Mfma<T, DP>;
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ BwdShared sh;
@@ -1569,6 +1569,11 @@ inline size_t sinkhorn_bwd_lds_bytes_t(int N, int DP, int elem, int G, int CH, b
   bytes += (2 * loc + 3 * loc + 68) * 4;                                  // lres, lout, dxs, dpw
   bytes += (size_t)(stream ? BWD_STREAM_SCRATCH : BWD_SCRATCH) * 4;
   return bytes;
+}
+
+template <typename T, int DP, bool STREAM, bool GEN>
+__global__ void __launch_bounds__(BWD_NT) sinkhorn_bwd_kernel(SinkBwdArgs a) {
+  sinkhorn_bwd_general<T, DP, STREAM, GEN>(a);
 }
 
 template <typename T, int DP, bool STREAM, bool GEN>

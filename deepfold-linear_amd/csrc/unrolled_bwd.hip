@@ -46,7 +46,7 @@ template <typename T, int DP>
 __global__ void __launch_bounds__(256) unrolled_prep_kernel(UnrPrepArgs p) {
   const int N = p.N, d = p.d;
   const int Np = ((N + 31) / 32) * 32;
-  sb_clear_steps(p.steps, p.B * p.H, N, p.K);
+  if (p.steps) sb_clear_steps(p.steps, p.B * p.H, N, p.K);
   const size_t e = (size_t)blockIdx.x * 256 + threadIdx.x;
   const size_t row = e / DP;
   const int c = (int)(e % DP);
@@ -78,6 +78,12 @@ __global__ void __launch_bounds__(256) unrolled_prep_kernel(UnrPrepArgs p) {
   static_cast<T*>(p.qt)[((size_t)bh * DP + c) * Np + i] = from_f32<T>(qv);
   static_cast<T*>(p.kt)[((size_t)bh * DP + c) * Np + i] = from_f32<T>(kv);
   p.gt[((size_t)bh * DP + c) * Np + i] = go;
+  if (p.go_hi) {
+    const T hi = from_f32<T>(go);
+    static_cast<T*>(p.go_hi)[row * DP + c] = hi;
+    static_cast<T*>(p.go_lo)[row * DP + c] = from_f32<T>(go - to_f32(hi));
+    static_cast<T*>(p.go_t)[((size_t)bh * DP + c) * Np + i] = hi;
+  }
   float part = go * oa;
 #pragma unroll
   for (int o = DP / 2; o >= 1; o >>= 1) part += __shfl_xor(part, o, WAVE);

@@ -163,3 +163,46 @@ def test_register_unrolled_gradients(B, H, N, d, K, lengths):
     o.backward(go.to(DEV))
     for k in names:
         assert_close_rel(p[k].grad.cpu().double().numpy(), want[k], 1e-4, "d" + k)
+
+
+@pytest.mark.parametrize("solver,iters,mode", [
+    ("fixed_point", 4, "reference"), ("fixed_point", 0, "reference"), ("cg", 20, "reference"), ("cg", 20, "analytic"),
+])
+@pytest.mark.parametrize("B,H,N,d,v_scale,geo,lengths,dtype,tol", [
+    (1, 2, 17, 32, 0.0, True, None, torch.float32, 1e-4),          # members without a tile
+    (2, 8, 300, 24, 0.0, False, [300, 161], torch.float32, 1e-4),  # three tiles a member; padded columns
+    (1, 4, 150, 32, 0.0, True, None, torch.bfloat16, 2e-2),
+    (1, 4, 90, 32, 60.0, True, None, torch.float32, 1e-3),         # row sums out of range: the general sweeps as a call
+])
+def test_register_ift_gradients(B, H, N, d, v_scale, geo, lengths, dtype, tol, solver, iters, mode):
+    from test_gpu_sinkhorn_bwd import compare, grad_inputs, run_gpu_bwd
+    from test_gpu_sinkhorn_fwd import make_inputs, oracle_inputs
+
+    print(f"case B{B} H{H} N{N} d{d} v{v_scale} geo={geo} {dtype} {solver} {iters} {mode}", flush=True)
+    inp = make_inputs(B, H, N, d, seed=N + d, eps=[1.0, 0.7] * (H // 2), pos_geo=geo)
+    go, gxc = grad_inputs(B, H, N, d, seed=N + 1, with_xc=lengths is None)
+    K, mask, kw = 6, None, {}
+    if lengths is not None:
+        mask = torch.zeros(B, N)
+        for b, n in enumerate(lengths):
+            mask[b, :n] = 1
+        go = go * mask[:, :, None]
+    oi = dict(oracle_inputs(inp, dtype))
+    if v_scale:
+        K = 1
+        v0 = v_scale * torch.randn(B, H, N, generator=torch.Generator().manual_seed(4))
+        kw["log_v_init"] = v0.to(DEV)
+        oi["log_v_init"] = v0.numpy()
+    got = run_gpu_bwd(inp, K, dtype, go, gxc, mask=mask, ift_solver=solver, ift_iters=iters, ift_mode=mode, **kw)
+    gx = None if gxc is None else gxc.numpy()
+    oi["K_iter"] = K
+    if mask is not None:
+        _, want = ref.backward_masked(dict(oi, mask=mask.numpy(), lam=1.0, r_0=10.0), go.numpy(), gx, mode=mode,
+                                      solver=solver, n_cg=iters, K_back=iters)
+    else:
+        fo = ref.forward(**oi)
+        if mode == "analytic":
+            want = ref.backward_analytic(oi, fo, go.numpy(), gx)
+        else:
+            want = ref.backward_reference(oi, fo, go.numpy(), gx, K_back=iters, solver=solver, n_cg=iters)
+    compare(got, want, tol, f"ift-{mode}-{solver}", skip=() if mask is None else ("pos_weight", "w_dist", "x_res"))
