@@ -164,12 +164,50 @@ template <typename T, int LD> struct Flight<T, LD, false> {
   }
 };
 
+// 16- and 8-byte global accesses without an alignment requirement beyond the element's.
+__device__ __forceinline__ uint4 ld16_any(const void* p) {
+  uint4 r;
+  __builtin_memcpy(&r, p, 16);
+  return r;
+}
+__device__ __forceinline__ uint2 ld8_any(const void* p) {
+  uint2 r;
+  __builtin_memcpy(&r, p, 8);
+  return r;
+}
+
+// Move the elements (ES bytes, 2 or 4) of W words down by s places, zeros from the top;
+// W words hold 4 or 8 elements.  s <= 0 and s >= the element count leave them as they are.
+template <int W, int ES>
+__device__ __forceinline__ void shift_down(unsigned (&w)[W], int s) {
+  constexpr int N = W * 4 / ES;
+  if (s < 0 || s >= N) s = 0;
+  if (ES == 2) {
+    const bool odd = s & 1;
+#pragma unroll
+    for (int i = 0; i < W; ++i) {
+      const unsigned hi = i + 1 < W ? w[i + 1] : 0u;
+      w[i] = odd ? (w[i] >> 16) | (hi << 16) : w[i];
+    }
+    s >>= 1;
+  }
+#pragma unroll
+  for (int bit = 1; bit < W; bit *= 2) {
+    const bool on = s & bit;
+#pragma unroll
+    for (int i = 0; i < W; ++i) w[i] = on ? (i + bit < W ? w[i + bit] : 0u) : w[i];
+  }
+}
+
 // Per-(query, key) bias of one lane's query row, in log2 units.
 //   DENSE / WINDOW: element type T, LOG2E * bias;  BINS: int32 bin -> pw2[bin] (pre-scaled).
 // row: element of key 0 of the lane's (clamped) query row; keys start at the
-// window offset for WINDOW.  FAST loads take 8 consecutive keys as 16-byte blocks
-// from a start clamped to [.., k_hi - 8]: keys past k_hi read another key's value,
-// which the -1e30 key mask of those keys swamps.
+// window offset for WINDOW.  FAST loads take 8 consecutive keys as 16-byte blocks of
+// any alignment (rows of an odd key count start anywhere; global memory takes
+// under-aligned 16-byte loads) from a start clamped to [.., k_hi - 8].  A group that
+// crosses k_hi is moved into place by tail8 before use (one step of a row; its keys
+// past k_hi read zero); a group wholly past k_hi holds other keys' values, which the
+// -1e30 key mask of those keys swamps.
 template <typename T, int BIAS>
 struct BiasRow {
   using BT = typename std::conditional<BIAS == ATTN_BIAS_BINS, int, T>::type;
@@ -178,7 +216,15 @@ struct BiasRow {
   __device__ __forceinline__ void load8(uint4 (&r)[BW], int key0, int k_hi) const {
     const int kc = min(key0, k_hi - 8);
 #pragma unroll
-    for (int w = 0; w < BW; ++w) r[w] = *reinterpret_cast<const uint4*>(row + kc + w * (16 / (int)sizeof(BT)));
+    for (int w = 0; w < BW; ++w) r[w] = ld16_any(row + kc + w * (16 / (int)sizeof(BT)));
+  }
+  __device__ __forceinline__ static void tail8(uint4 (&r)[BW], int key0, int k_hi) {
+    union { uint4 u[BW]; unsigned w[4 * BW]; } x;
+#pragma unroll
+    for (int w = 0; w < BW; ++w) x.u[w] = r[w];
+    shift_down<4 * BW, (int)sizeof(BT)>(x.w, key0 - (k_hi - 8));
+#pragma unroll
+    for (int w = 0; w < BW; ++w) r[w] = x.u[w];
   }
   __device__ __forceinline__ float elem(int key, int k_hi, const float* pw2) const {
     const BT v = row[min(key, k_hi - 1)];
@@ -406,6 +452,7 @@ __global__ void __launch_bounds__((Eng<T, DP, WIN>::NT)) attn_fwd2_kernel(AttnAr
     for (int j = 0; j < SPW; ++j) {
       const int kl = 32 * (ks + KS * j);  // local row of this step
       if (c0 + kl >= k_hi) break;
+      if (HASB && FAST && c0 + kl + 32 > k_hi) BR::tail8(bcur[j], c0 + kl + 8 * g, k_hi);
       typename M::Frag kf0, kf1;
       const int pr = kl + perm_row(lane, 0);
       M::load(kf0, Ks + (size_t)pr * RS, lane);
@@ -719,6 +766,7 @@ __global__ void __launch_bounds__((Eng<T, DP, WIN>::NT)) attn_bwd_q2_kernel(Attn
     for (int j = 0; j < SPW; ++j) {
       const int kl = 32 * (ks + KS * j);
       if (c0 + kl >= k_hi) break;
+      if (HASB && FAST && c0 + kl + 32 > k_hi) BR::tail8(bcur[j], c0 + kl + 8 * g, k_hi);
       const int pr = kl + perm_row(lane, 0);
       typename M::Frag f0, f1;
       M::load(f0, Ks + (size_t)pr * RS, lane);
@@ -761,7 +809,7 @@ __global__ void __launch_bounds__((Eng<T, DP, WIN>::NT)) attn_bwd_q2_kernel(Attn
         if (FAST && key0 + 8 <= k_hi) {
 #pragma unroll
           for (int w = 0; w < (sizeof(T) == 2 ? 1 : 2); ++w)
-            *reinterpret_cast<uint4*>(drow + key0 + w * (16 / (int)sizeof(T))) = o.u[w];
+            __builtin_memcpy(drow + key0 + w * (16 / (int)sizeof(T)), &o.u[w], 16);  // any alignment, as the bias
         } else {
 #pragma unroll
           for (int e = 0; e < 8; ++e)
@@ -850,11 +898,11 @@ struct KVBias {
   __device__ static __forceinline__ void load(Raw& r, const BT* row, int key, int k_hi) {
     if (FAST) {
       if (BF) {
-        const uint2 v = *reinterpret_cast<const uint2*>(row + min(key, k_hi - 4));
+        const uint2 v = ld8_any(row + min(key, k_hi - 4));
         r.w[0] = v.x;
         r.w[1] = v.y;
       } else {
-        const uint4 v = *reinterpret_cast<const uint4*>(row + min(key, k_hi - 4));
+        const uint4 v = ld16_any(row + min(key, k_hi - 4));
         r.w[0] = v.x; r.w[1] = v.y; r.w[2] = v.z; r.w[3] = v.w;
       }
     } else {
@@ -1088,6 +1136,10 @@ __global__ void __launch_bounds__(512) attn_bwd_kv2_kernel(AttnArgs a) {
         if (FAST) {
           r0 = bcur[j][0];
           r1 = bcur[j][1];
+          if (kt + 16 > bk_hi) {  // the sequence's last key tile: four keys that cross its end are moved into place
+            shift_down<KB::NW, (int)sizeof(typename KB::BT)>(r0.w, bkey - (bk_hi - 4));
+            shift_down<KB::NW, (int)sizeof(typename KB::BT)>(r1.w, bkey - (bk_hi - 4));
+          }
         } else {
           KB::load(r0, bias_row(qp + perm_row(lane, 0)), bkey, bk_hi);
           KB::load(r1, bias_row(qp + perm_row(lane, 1)), bkey, bk_hi);

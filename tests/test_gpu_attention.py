@@ -87,9 +87,9 @@ def test_diffusion_forward_backward(B, H, N, D, dtype):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("N,D", [(160, 24), (150, 20), (96, 64)])
 def test_diffusion_pair_bias_and_gate(N, D, dtype):
-    """cfg3-shaped extension (smaller N): dense pair bias + sigmoid gate.  N = 150 is not
-    a multiple of 8, so the kernels take their element-load staging (and D = 20 is not a
-    whole number of 16-byte bf16 blocks); D = 64 runs the 64-wide head instantiations."""
+    """cfg3-shaped extension (smaller N): dense pair bias + sigmoid gate.  D = 20 is
+    not a whole number of 16-byte bf16 blocks, so the kernels take their element-load
+    staging; D = 64 runs the 64-wide head instantiations."""
     from deepfold_amd import flash_diffusion_attn
 
     B, H = 1, 4
@@ -103,6 +103,40 @@ def test_diffusion_pair_bias_and_gate(N, D, dtype):
     t = tol(dtype)
     check("O", out, o_ref, t)
     for k in ("Q", "K", "V", "pair_bias", "gate"):
+        check("d" + k, g[k], g_ref[k], t)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("kind", ["dense", "bins", "window"])
+@pytest.mark.parametrize("N", [7, 8, 9, 33, 63, 129, 147, 262])
+def test_bias_rows_of_any_alignment(N, kind, dtype):
+    """Whole 16-byte heads with a bias whose rows start at any element: key counts that leave
+    1 .. 7 keys in the last group of 8 (and of 4, dK/dV pass), one key in the last tile of 16
+    and chunk, and N = 7, which keeps the element loads; a bias tensor that is itself one
+    element off 16-byte alignment."""
+    from deepfold_amd import flash_atom_attn, flash_diffusion_attn
+
+    B, H, D = 2, 2, 32
+    Q, K, V = (rnd(B, H, N, D, seed=s, dtype=dtype) for s in (51, 52, 53))
+    go = rnd(B, H, N, D, seed=54, dtype=dtype)
+    if kind == "window":
+        inp = dict(Q=Q, K=K, V=V, mask=None, window_bias=rnd((N + 31) // 32, H, 32, 128, seed=55, dtype=dtype))
+        fn, rfn, wrt = flash_atom_attn, ref.atom_attn, ("Q", "K", "V", "window_bias")
+    elif kind == "dense":
+        bias = torch.empty(B * H * N * N + 1, dtype=dtype, device=DEV)[1:].view(B, H, N, N)
+        inp = dict(Q=Q, K=K, V=V, pos_weight=None, pos_bins=None,
+                   pair_bias=bias.copy_(rnd(B, H, N, N, seed=55, dtype=dtype)))
+        fn, rfn, wrt = flash_diffusion_attn, ref.diffusion_attn, ("Q", "K", "V", "pair_bias")
+    else:
+        bins = torch.randint(0, 68, (B, N, N), generator=torch.Generator().manual_seed(56), dtype=torch.int32)
+        inp = dict(Q=Q, K=K, V=V, pos_weight=rnd(H, 68, seed=57), pos_bins=bins)
+        fn, rfn, wrt = flash_diffusion_attn, ref.diffusion_attn, ("Q", "K", "V", "pos_weight")
+    out, g = run_gpu(fn, inp, go, wrt)
+    o_ref, g_ref = ref.grads(rfn, {k: (v.double().cpu() if v is not None and v.is_floating_point() else v)
+                                   for k, v in inp.items()}, go.double(), wrt)
+    t = tol(dtype)
+    check("O", out, o_ref, t)
+    for k in wrt:
         check("d" + k, g[k], g_ref[k], t)
 
 
