@@ -34,8 +34,12 @@ struct Eng {
   static constexpr int KS = 2;                       // waves per resident tile
   static constexpr int NW = RT * KS;
   static constexpr int NT = NW * WAVE;
-  static constexpr int CH0 = RB <= 64 ? 256 : (RB <= 128 ? 128 : 64);
-  static constexpr int CH = (WIN && CH0 > 128) ? 128 : CH0;  // streamed rows per chunk
+  // Streamed rows per chunk.  128, not 256, where rows take 64 bytes (bf16, d <= 32): the two
+  // buffers of 256 rows took 115 KB (dQ) and 150 KB (dK/dV) of LDS, one workgroup a CU and two
+  // waves a SIMD for passes that wait on the bias stream; at half of it two workgroups fit.
+  // Dense bias, B 4, H 16, N 1024, d 24 (134 MB a read): forward 44.1 -> 40.9, dQ (reads the
+  // bias, writes its gradient) 78.5 -> 62.8, dK/dV 78.1 -> 59.6 us.
+  static constexpr int CH = RB <= 128 ? 128 : 64;
   static constexpr int SPC = CH / 32;                // 32-row steps per chunk
   static constexpr int SPW = SPC / KS;               // steps per wave per chunk
   static constexpr int CB = DP / VEC;                // 16-byte blocks per row
