@@ -424,6 +424,13 @@ __device__ __forceinline__ void scaled_bwd(const Args& a, General general) {
       const float ac_c = ok_c ? fast_exp2(lz_c) : 0.f, bc_c = ok_c ? fast_exp2(-vc_c) : 0.f;
       const float gv_c = has_q ? reg_sum<SB_NW>(scratch, qc) : 0.f;
       float zu_c = 0.f, zv_c = gv_c;
+      // No poll writes the entries past the last valid one: zero them in this wave's streamed tiles,
+      // where they hold the exponent terms' NEG_BIG (the gradient pass multiplies them by factors of
+      // up to 2^SB_MAX, past the float range)
+      for (int e = lane; e < 16 * KSL; e += WAVE) {
+        const int i = (wave + SB_NW * (e >> 4)) * 16 + (e & 15);
+        if (i >= n) wY[i] = wZ[i] = 0.f;
+      }
       auto take0 = [&](float* w) {
         return [w](int, int i, float v, bool ok) {
           w[i] = ok ? v : 0.f;

@@ -206,3 +206,43 @@ def test_register_ift_gradients(B, H, N, d, v_scale, geo, lengths, dtype, tol, s
         else:
             want = ref.backward_reference(oi, fo, go.numpy(), gx, K_back=iters, solver=solver, n_cg=iters)
     compare(got, want, tol, f"ift-{mode}-{solver}", skip=() if mask is None else ("pos_weight", "w_dist", "x_res"))
+
+
+@pytest.mark.parametrize("solver,iters,mode", [
+    ("fixed_point", 4, "reference"), ("fixed_point", 0, "reference"), ("fixed_point", 20, "analytic"),
+    ("cg", 10, "reference"),
+])
+@pytest.mark.parametrize("geo,dtype,tol", [(False, torch.float32, 1e-4), (True, torch.float32, 1e-4),
+                                           (True, torch.bfloat16, 2e-2)])
+def test_register_ift_large_row_sums(geo, dtype, tol, solver, iters, mode):
+    """Row sums near the top of the register form's range (log Z of 20 nats, the range ends at 22.2) and a
+    last tile that the sequence does not fill: the entries past its end take part in no sum."""
+    from test_gpu_sinkhorn_bwd import compare, grad_inputs, run_gpu_bwd
+    from test_gpu_sinkhorn_fwd import make_inputs, oracle_inputs
+
+    B, H, N, d, K = 1, 2, 90, 32, 1
+    print(f"case geo={geo} {dtype} {solver} {iters} {mode}", flush=True)
+    inp = make_inputs(B, H, N, d, seed=91, eps=[1.0, 1.0], pos_geo=geo)
+    v0 = torch.full((B, H, N), -90.0)
+    go, gxc = grad_inputs(B, H, N, d, seed=92, with_xc=True)
+    oi = dict(oracle_inputs(inp, dtype), log_v_init=v0.numpy(), K_iter=K)
+    fo = ref.forward(**oi)
+    logz = []
+    for h in range(H):
+        z = ref._plan_pieces(oi["Q"][0, h], oi["K"][0, h], oi["x_res"][0], oi["pos_weight"][h],
+                             None if oi["pos_bins"] is None else oi["pos_bins"][0], oi["w_dist"][h], 10.0,
+                             oi["eps"][h], fo["log_u"][0, h], fo["log_v"][0, h])
+        logz.append(z["logZ"])
+        # v + column LSE = log nu - eps / lam v: both factors inside the range, so that no group leaves the form
+        assert np.max(np.abs(oi["log_nu"][0, h] - fo["log_v"][0, h])) < MAX_DRIFT
+    assert np.max(logz) < MAX_DRIFT and np.max(logz) > 19.7  # 2^128 / 1e30 in nats: the product that overflowed
+    got = run_gpu_bwd(inp, K, dtype, go, gxc, ift_solver=solver, ift_iters=iters, ift_mode=mode,
+                      log_v_init=v0.to(DEV))
+    for k, v in got.items():
+        assert np.isfinite(v).all(), k
+    if mode == "analytic":
+        want = ref.backward_analytic(oi, fo, go.numpy(), gxc.numpy())
+    else:
+        want = ref.backward_reference(oi, fo, go.numpy(), gxc.numpy(), K_back=iters, solver=solver, n_cg=iters)
+    # (the analytic oracle solves the system exactly: 20 sweeps leave a share of kappa^40 = 2^-40)
+    compare(got, want, tol, f"large-row-sums-{mode}-{solver}")
