@@ -83,7 +83,7 @@ __global__ void __launch_bounds__(256) balanced_prep_kernel(BalPrepArgs p) {
     p.gt[((size_t)bh * DP + c) * Np + i] = gv;
   }
   if (c < 3) p.gxs[((size_t)bh * 3 + c) * Np + i] = (ok && p.gxc) ? p.gxc[((size_t)bh * N + i) * 3 + c] : 0.f;
-  if (c < 3 && h == 0) p.xs[((size_t)b * 3 + c) * Np + i] = i < N ? p.x[((size_t)b * N + i) * 3 + c] : 0.f;
+  if (c < 3 && h == 0) p.xs[((size_t)b * 3 + c) * Np + i] = ok ? p.x[((size_t)b * N + i) * 3 + c] : 0.f;
   if (c == 0) {
     float D = 0.f;
     if (ok) {

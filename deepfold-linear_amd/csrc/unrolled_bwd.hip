@@ -42,6 +42,7 @@ constexpr int UNR_MAX_LOCAL = 16 * UNR_MAXT_ANY * UNR_NW;  // rows of a stripe (
 
 // Prep: one thread per (b, h, i, c), c < DP.  fp32 copies of Q, K, V, gO and gO^T,
 // D, grad x_c, coordinates; dG = sigma(1 - sigma) O dO (flash_sinkhorn_attn.py:278-292).
+// Masked rows are zero throughout: whatever the caller's padding holds reaches no sum.
 template <typename T, int DP>
 __global__ void __launch_bounds__(256) unrolled_prep_kernel(UnrPrepArgs p) {
   const int N = p.N, d = p.d;
@@ -88,7 +89,7 @@ __global__ void __launch_bounds__(256) unrolled_prep_kernel(UnrPrepArgs p) {
 #pragma unroll
   for (int o = DP / 2; o >= 1; o >>= 1) part += __shfl_xor(part, o, WAVE);
   if (c < 3) p.gxs[((size_t)bh * 3 + c) * Np + i] = (ok && p.grad_xc) ? p.grad_xc[((size_t)bh * N + i) * 3 + c] : 0.f;
-  if (c < 3 && h == 0) p.xs[((size_t)b * 3 + c) * Np + i] = (p.x && i < N) ? p.x[((size_t)b * N + i) * 3 + c] : 0.f;
+  if (c < 3 && h == 0) p.xs[((size_t)b * 3 + c) * Np + i] = (p.x && ok) ? p.x[((size_t)b * N + i) * 3 + c] : 0.f;
   if (c == 0) {
     if (ok && p.grad_xc)
       for (int t = 0; t < 3; ++t) part += p.grad_xc[((size_t)bh * N + i) * 3 + t] * p.xc[((size_t)bh * N + i) * 3 + t];

@@ -246,3 +246,45 @@ def test_register_ift_large_row_sums(geo, dtype, tol, solver, iters, mode):
         want = ref.backward_reference(oi, fo, go.numpy(), gxc.numpy(), K_back=iters, solver=solver, n_cg=iters)
     # (the analytic oracle solves the system exactly: 20 sweeps leave a share of kappa^40 = 2^-40)
     compare(got, want, tol, f"large-row-sums-{mode}-{solver}")
+
+
+@pytest.mark.parametrize("op,geo", [("fixed_point", False), ("fixed_point", True), ("cg", False), ("cg", True),
+                                    ("unrolled", False), ("unrolled", True), ("balanced", True)])
+def test_gradients_ignore_padded_inputs(op, geo):
+    """What padded rows hold, NaN included, changes no output and no gradient."""
+    from deepfold_amd import balanced_sinkhorn_transport_dual, flash_sinkhorn_attn
+
+    print(f"case {op} geo={geo}", flush=True)
+    B, H, N, d, lengths = 2, 4, 90, 32, [83, 50]
+    t = _uot(B, H, N, d, 5, 17, 0.0, lengths)
+    g = torch.Generator().manual_seed(18)
+    bins = torch.randint(0, 68, (B, N, N), generator=g, dtype=torch.int32).to(DEV) if geo else None
+    t.update(pos_weight=0.3 * torch.randn(H, 68, generator=g), w_dist=torch.rand(H, generator=g),
+             alpha=torch.full((H,), -1.0), r=torch.full((H,), 10.0))
+    m = t["mask"].to(DEV)
+    gx = torch.randn(B, H, N, 3, generator=g).to(DEV) * m[:, None, :, None]
+    go = torch.randn(B, N, H * d, generator=g).to(DEV) * m[:, :, None]
+    runs = []
+    for fill in (0.0, float("nan")):
+        c = {k: v.to(DEV).clone() for k, v in t.items()}
+        for k in ("Q", "K", "V", "G"):
+            c[k] = torch.where(m[:, None, :, None] > 0, c[k], torch.full_like(c[k], fill))
+        c["x_res"] = torch.where(m[:, :, None] > 0, c["x_res"], torch.full_like(c["x_res"], fill))
+        if op == "balanced":
+            names = ("Q", "K", "x_res", "V", "alpha", "r")
+            p = {k: c[k].requires_grad_(True) for k in names}
+            out = balanced_sinkhorn_transport_dual(p["Q"], p["K"], p["x_res"], p["V"], c["eps"], p["alpha"], p["r"],
+                                                   K_iter=5, mask=m)
+            seeds = [gx, go.view(B, N, H, d).permute(0, 2, 1, 3).contiguous()]
+        else:
+            names = ("Q", "K", "V", "G", "x_res", "log_mu", "log_nu") + (("w_dist",) if geo else ())
+            p = {k: c[k].requires_grad_(True) for k in names}
+            kw = {"ift_mode": "unrolled"} if op == "unrolled" else {"ift_solver": op, "ift_iters": 6}
+            out = flash_sinkhorn_attn(p["Q"], p["K"], p["V"], p["G"], p["x_res"], c["pos_weight"], bins, c["eps"],
+                                      p.get("w_dist"), p["log_mu"], p["log_nu"], K_iter=5, mask=m, **kw)[:2]
+            seeds = [go, gx]
+        grads = torch.autograd.grad(list(out), list(p.values()), seeds)
+        runs.append(dict(zip(names, grads), **{f"out{i}": o.detach() for i, o in enumerate(out)}))
+    for k, want in runs[0].items():
+        assert torch.isfinite(want).all(), k
+        assert torch.equal(runs[1][k], want), k
