@@ -491,10 +491,9 @@ template <int DP>
 __global__ void __launch_bounds__(BAL_NT) balanced_bwd_kernel(BalBwdArgs a) {
   balanced_general<DP>(a);
 }
-// Register form (scaled_bwd.h); the general sweeps are a call, so that they cost its sweeps no registers.
-__device__ __attribute__((noinline)) void balanced_general_call(BalBwdArgs a) { balanced_general<32>(a); }
+// Register form (scaled_bwd.h).
 __global__ void __launch_bounds__(SB_NT) balanced_scaled_kernel(BalBwdArgs a) {
-  scaled_bwd<float, true>(a, [](const BalBwdArgs& x) { balanced_general_call(x); });
+  if (scaled_bwd<float, true>(a)) balanced_general<32>(fresh_args<BalBwdArgs>());
 }
 
 size_t scaled_step_words(int N) { return sb_step_words(N); }

@@ -77,10 +77,25 @@ inline bool sb_fits(int N, int DP, int G, int K, bool bal, size_t limit) {
   return DP == 32 && K >= 1 && K <= SB_KMAX && reg_fits(N, G) && sb_lds_bytes(N, G, K, bal) + 2048 <= limit;
 }
 
+// The kernel's argument struct (its only parameter) for the general sweeps, read anew from where the
+// launch put it: nothing that they read is held in registers through the register form.
+template <typename Args> __device__ __forceinline__ const Args& fresh_args() {
+  typedef const __attribute__((address_space(4))) Args* Place;
+  Place p = (Place)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const Args*)p;
+}
+
 // T: input type of Q, K and of the gradients; GEN: the cost may carry bins or geometry (always in
-// the balanced mode); general(a): the general sweeps, for a group whose factors are out of range.
-template <typename T, bool GEN, typename Args, typename General>
-__device__ __forceinline__ void scaled_bwd(const Args& a, General general) {
+// the balanced mode).  Returns, uniformly over the group, whether the general sweeps have to run: a group
+// whose factors are out of range, and a member that owns nothing (they do its part of the zeroing).
+// The kernels inline them behind this one test, where nothing of the register form is live.  As a call
+// with the arguments by value they read sizes, pointers and branch conditions per lane from its stack.
+// Every group out of range, us, in a kernel of their own / as a call / so: implicit, bf16, 16 heads of
+// 768 tokens, 20 CG steps 201 / 530 / 207; unrolled, fp32, 16 heads of 300 with bins and geometry
+// 1054 / 1645 / 1070; balanced, 16 heads of 256, K 20 309 / 325 / 314.
+template <typename T, bool GEN, typename Args>
+__device__ __forceinline__ bool scaled_bwd(const Args& a) {
   constexpr bool BAL = is_bal<Args>::value, IFT = is_ift<Args>::value, UNR = !BAL && !IFT;
   constexpr int DP = 32, NC = DP / 16;
   using MQ = Mfma<T, DP>;
@@ -89,7 +104,7 @@ __device__ __forceinline__ void scaled_bwd(const Args& a, General general) {
   __shared__ int s_flagp[2], s_tmp, s_flag, s_local, s_ok, s_cnt;
   __shared__ float sscal[2 * SB_NW], s_red[2 * SB_NW];
   int grp, member;
-  if (!group_of(a.B * a.H, a.G, grp, member)) return;
+  if (!group_of(a.B * a.H, a.G, grp, member)) return false;
   const int b = grp / a.H, h = grp % a.H;
   const int N = a.N, d = a.d, BH = a.B * a.H;
   int K = 0;  // (IFT: no recorded iterations)
@@ -135,7 +150,7 @@ __device__ __forceinline__ void scaled_bwd(const Args& a, General general) {
   int t0, t1;
   stripe(n_tiles, member, a.G, t0, t1);
   const int nr = t1 - t0, r_lo = t0 * 16;
-  if (n == 0 || nr <= 0) { general(a); return; }  // owns nothing: its part of the zeroing only
+  if (n == 0 || nr <= 0) return true;
   // ---- factors of my stripe, and whether they are in range
   const float eps = a.eps[h];
   float w_bal = 0.f, kappa = 1.f, wd = 0.f, lm2 = 0.f;
@@ -251,8 +266,8 @@ __device__ __forceinline__ void scaled_bwd(const Args& a, General general) {
       if (!got) s_flag = 1;
     }
     __syncthreads();
-    if (s_flag) return;
-    if (!s_ok) { general(a); return; }
+    if (s_flag) return false;
+    if (!s_ok) return true;
   }
   const bool local = s_local != 0;
   // rows past the last valid tile belong to no stripe: zeroed here (row i by member i % G)
@@ -908,6 +923,7 @@ __device__ __forceinline__ void scaled_bwd(const Args& a, General general) {
   if (ksg == 2) run(std::integral_constant<int, 2>{});
   else if (ksg == 4) run(std::integral_constant<int, 4>{});
   else run(std::integral_constant<int, 6>{});
+  return false;
 }
 
 }  // namespace dfl

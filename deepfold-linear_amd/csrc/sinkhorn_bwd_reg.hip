@@ -11,11 +11,8 @@
 namespace dfl {
 
 template <typename T, bool GEN>
-__device__ __attribute__((noinline)) void ift_general_call(SinkBwdArgs a) { sinkhorn_bwd_general<T, 32, false, GEN>(a); }
-
-template <typename T, bool GEN>
 __global__ void __launch_bounds__(SB_NT) ift_scaled_kernel(IftBwdArgs a) {
-  scaled_bwd<T, GEN>(a, [](const IftBwdArgs& x) { ift_general_call<T, GEN>(x); });
+  if (scaled_bwd<T, GEN>(a)) sinkhorn_bwd_general<T, 32, false, GEN>(fresh_args<IftBwdArgs>());
 }
 
 template <typename T, bool GEN>

@@ -967,14 +967,10 @@ template <typename T, int DP, bool GEN, int OPS>
 __global__ void __launch_bounds__(UNR_NT) unrolled_bwd_kernel(UnrBwdArgs a) {
   unrolled_general<T, DP, GEN, OPS>(a);
 }
-// Register form (scaled_bwd.h); the general sweeps are a call, so that they cost its sweeps no registers.
-template <typename T, bool GEN>
-__device__ __attribute__((noinline)) void unrolled_general_call(UnrBwdArgs a) {
-  unrolled_general<T, 32, GEN, UNR_OPS_GLOBAL>(a);
-}
+// Register form (scaled_bwd.h).
 template <typename T, bool GEN>
 __global__ void __launch_bounds__(SB_NT) unrolled_scaled_kernel(UnrBwdArgs a) {
-  scaled_bwd<T, GEN>(a, [](const UnrBwdArgs& x) { unrolled_general_call<T, GEN>(x); });
+  if (scaled_bwd<T, GEN>(a)) unrolled_general<T, 32, GEN, UNR_OPS_GLOBAL>(fresh_args<UnrBwdArgs>());
 }
 
 size_t unrolled_bwd_lds_bytes(int N, int DP, int elem, int ops) {
