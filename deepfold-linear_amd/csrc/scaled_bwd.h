@@ -87,7 +87,7 @@ template <typename Args> __device__ __forceinline__ const Args& fresh_args() {
 }
 
 // T: input type of Q, K and of the gradients; GEN: the cost may carry bins or geometry (always in
-// the balanced mode).  Returns, uniformly over the group, whether the general sweeps have to run: a group
+// the balanced mode).  Returns, uniformly over the workgroup, whether the general sweeps have to run: a group
 // whose factors are out of range, and a member that owns nothing (they do its part of the zeroing).
 // The kernels inline them behind this one test, where nothing of the register form is live.  As a call
 // with the arguments by value they read sizes, pointers and branch conditions per lane from its stack.

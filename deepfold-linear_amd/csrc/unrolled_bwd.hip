@@ -967,10 +967,12 @@ template <typename T, int DP, bool GEN, int OPS>
 __global__ void __launch_bounds__(UNR_NT) unrolled_bwd_kernel(UnrBwdArgs a) {
   unrolled_general<T, DP, GEN, OPS>(a);
 }
-// Register form (scaled_bwd.h).
+// Register form (scaled_bwd.h).  A bf16 group out of its range keeps resident operands: 2x8 heads of 768
+// tokens, K 50, 1472 us with operands from L2, 762 with resident ones (753 in a kernel of their own).
+template <typename T> constexpr int scaled_ops = sizeof(T) == 2 ? UNR_OPS_RES : UNR_OPS_GLOBAL;
 template <typename T, bool GEN>
 __global__ void __launch_bounds__(SB_NT) unrolled_scaled_kernel(UnrBwdArgs a) {
-  if (scaled_bwd<T, GEN>(a)) unrolled_general<T, 32, GEN, UNR_OPS_GLOBAL>(fresh_args<UnrBwdArgs>());
+  if (scaled_bwd<T, GEN>(a)) unrolled_general<T, 32, GEN, scaled_ops<T>>(fresh_args<UnrBwdArgs>());
 }
 
 size_t unrolled_bwd_lds_bytes(int N, int DP, int elem, int ops) {
@@ -1052,10 +1054,11 @@ static hipError_t launch_unr_dt(const UnrBwdArgs& a, int DP, size_t lds, hipStre
 // The register form where the stripes and the iterations' vectors fit (limit: LDS of a workgroup).
 hipError_t launch_unrolled_bwd(const UnrBwdArgs& a, bool bf16_in, int DP, size_t lds, size_t limit, hipStream_t stream,
                                bool coop, int ops) {
-  if (sb_fits(a.N, DP, a.G, a.K, false, limit - UNR_STATIC)) {
+  const size_t lds_general =
+      bf16_in ? unrolled_bwd_lds_bytes(a.N, DP, 2, scaled_ops<bf16>) : unrolled_bwd_lds_bytes(a.N, DP, 4, scaled_ops<float>);
+  if (sb_fits(a.N, DP, a.G, a.K, false, limit - UNR_STATIC) && lds_general <= limit - UNR_STATIC) {
     const bool gen = (a.bins8 && a.pos_w) || (a.has_geo && a.w_dist);
-    const size_t need = std::max(sb_lds_bytes(a.N, a.G, a.K, false),
-                                 unrolled_bwd_lds_bytes(a.N, DP, bf16_in ? 2 : 4, UNR_OPS_GLOBAL));
+    const size_t need = std::max(sb_lds_bytes(a.N, a.G, a.K, false), lds_general);
     if (bf16_in)
       return gen ? launch_unr_k(unrolled_scaled_kernel<bf16, true>, a, need, stream, coop)
                  : launch_unr_k(unrolled_scaled_kernel<bf16, false>, a, need, stream, coop);

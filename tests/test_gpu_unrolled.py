@@ -80,7 +80,7 @@ CASES = [
     (2, 3, 70, 32, 3, [0.5, 1.0, 2.0], [70, 41], True, torch.float32, 1e-4),
     (1, 2, 48, 64, 5, [0.7, 1.3], None, False, torch.bfloat16, 2e-2),
     (1, 2, 300, 32, 4, [0.5, 1.0], [290], False, torch.float32, 1e-4),        # several tiles per member
-    # bf16 with d <= 32: Q and K resident in LDS (swizzled, transposed reads)
+    # bf16 with d <= 32
     (2, 3, 70, 32, 5, [0.5, 1.0, 2.0], [70, 41], False, torch.bfloat16, 2e-2),
     (1, 2, 300, 32, 4, [0.5, 1.0], [290], False, torch.bfloat16, 2e-2),
 ]
@@ -175,19 +175,20 @@ def _check(vg, L, vr, gr, tol):
 
 
 # (2, 8, 768, ...) is the headline layout (B2 H8 N768, n_b = [501, 759]: two and three
-# resident tiles per member, Q and K resident in LDS); at N = 832 resident operands would
-# need 166752 bytes of LDS (over 160 KiB), so that case reads Q and K from L2
+# resident tiles per member, the plan in registers); N = 832 is past the register form, and
+# resident operands would need 166752 bytes of LDS (over 160 KiB) there: Q and K from L2
 @pytest.mark.parametrize("B,H,N,d,K,lens", [(2, 4, 96, 32, 6, [96, 61]), (1, 2, 300, 24, 4, [290]),
                                              (2, 8, 768, 32, 3, [501, 759]), (1, 2, 832, 32, 3, [829])])
 def test_unrolled_content_only_bf16(B, H, N, d, K, lens):
     """The content-only cost (the build the headline workload runs) with bf16 inputs
-    at d <= 32 (Q and K resident in LDS)."""
+    at d <= 32."""
     print(f"case content-only B{B} H{H} N{N} d{d} K{K}", flush=True)
     _check(*_content_only(B, H, N, d, K, lens, torch.bfloat16), 2e-2)
 
 
 # B*H = 64 -> 4 members per head: 5-6 resident tiles per member (strided wave mapping,
-# two tiles a wave on some SIMDs) and 8-10 (whole tiles per wave); fp32 reads Q and K from L2
+# two tiles a wave on some SIMDs) and 8-10 (whole tiles per wave), more than the register
+# form holds: the general sweeps, bf16 with Q and K resident in LDS, fp32 with both from L2
 @pytest.mark.parametrize("N,lens,dtype,tol", [
     (384, [384, 350, 300, 330], torch.bfloat16, 2e-2),
     (640, [640, 600, 560, 530], torch.bfloat16, 2e-2),
@@ -200,6 +201,36 @@ def test_unrolled_many_tiles_per_member(N, lens, dtype, tol):
 
 @pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-4), (torch.bfloat16, 2e-2)])
 def test_unrolled_exact_factor_path(dtype, tol):
-    """Sweeps whose exponential ratio leaves the factored range take the exact path."""
+    """Sweeps whose exponential ratio leaves the factored range take the exact path (the groups
+    are out of the register form's range too: its kernel runs the general sweeps)."""
     print(f"case extreme marginals {dtype}", flush=True)
     _check(*_content_only(2, 2, 96, 32, 4, [96, 61], dtype, extreme=True), tol)
+
+
+# (1, 2, 96): groups that leave the register form inside its kernel; (4, 16, 384): six resident
+# tiles a member, the general sweeps in a kernel of their own, bf16 with resident Q and K
+@pytest.mark.parametrize("extreme", [False, True])
+@pytest.mark.parametrize("B,H,N,lens,K,dtype,tol", [
+    (1, 2, 96, [90], 4, torch.float32, 1e-4),
+    (1, 2, 96, [90], 4, torch.bfloat16, 2e-2),
+    (4, 16, 384, [384, 350, 300, 330], 3, torch.bfloat16, 2e-2),
+])
+def test_unrolled_general_sweeps_full_cost(B, H, N, lens, K, dtype, tol, extreme):
+    """Bins and geometry in the general sweeps, with and without marginals that put the exponential
+    ratio outside the factored range."""
+    print(f"case full cost B{B} H{H} N{N} K{K} {dtype} extreme={extreme}", flush=True)
+    t, bins, e, mask, wo, wx = _inputs(B, H, N, 32, seed=N + 5, eps=[0.5, 1.0] * (H // 2), lens=lens)
+    if extreme:
+        t["lmu"][..., :3] = -70.0
+        t["lnu"][..., 5:8] = -70.0
+    if dtype == torch.bfloat16:
+        for k in ("Q", "K", "V", "G"):
+            t[k] = t[k].to(torch.bfloat16).float()
+    vr, gr = _oracle(t, bins, e, mask, wo, wx, K)
+    vg, gg = _gpu(t, bins, e, mask, wo, wx, K, dtype)
+    for k in ("o", "xc", "lu", "lv"):
+        assert_close_rel(vg[k].detach().float().cpu().numpy(), vr[k].detach().numpy(), tol, k)
+    for k, want in gr.items():
+        got = gg[k].float().cpu().numpy()
+        assert np.isfinite(got).all(), k
+        assert_close_rel(got, want.numpy(), tol, f"grad {k}")
