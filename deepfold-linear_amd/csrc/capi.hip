@@ -691,6 +691,40 @@ size_t dfl_sinkhorn_bias_workspace_size(int B, int H, int N) {
   return 2 * (size_t)B * H * np * np * 4 + (bias_mat_offset(B, H, N) - dfl_sinkhorn_workspace_size(B, H, N));
 }
 
+// How dfl_sinkhorn_bwd runs a shape: LDS chunk, storage and LDS bytes, and whether the plan stays in
+// registers (where the stripes fit the register tiles).
+namespace {
+struct BwdPlan {
+  int G, CH;
+  bool stream, reg;
+  size_t lds;
+};
+BwdPlan bwd_plan(int B, int H, int N, int DP, int dtype, int storage) {
+  BwdPlan r;
+  r.G = group_size(B, H, N);
+  const int elem = dtype == DFL_BF16 ? 2 : 4;
+  r.CH = ((N + 31) / 32) * 32 < 256 ? ((N + 31) / 32) * 32 : 256;  // streamed rows per LDS chunk
+  r.lds = dfl::sinkhorn_bwd_lds_bytes(N, DP, elem, r.G, r.CH, false);
+  r.stream = storage == DFL_STORAGE_STREAM || (storage == DFL_STORAGE_AUTO && r.lds > LDS_LIMIT);
+  if (r.stream) {
+    // the largest chunk (multiple of 32 rows) whose staging fits next to the stripes
+    for (; r.CH > 32 && dfl::sinkhorn_bwd_lds_bytes(N, DP, elem, r.G, r.CH, true) > LDS_LIMIT; r.CH -= 32) {
+    }
+    r.lds = dfl::sinkhorn_bwd_lds_bytes(N, DP, elem, r.G, r.CH, true);
+  }
+  r.reg = !r.stream && storage == DFL_STORAGE_AUTO && dfl::sinkhorn_bwd_reg_fits(N, DP, r.G, r.lds, LDS_LIMIT);
+  return r;
+}
+}  // namespace
+
+// With the plan in registers the bias is evaluated once an element anyway, and a group that leaves that
+// form is no faster with the matrices: 16 heads of 768 tokens, 20 CG steps, all out of range, 425 us with
+// them (before the register form) and 406 without, 7 and 20 fixed-point steps 440 and 419, 707 and 664.
+size_t dfl_sinkhorn_bwd_bias_workspace_size(int B, int H, int N, int d, int dtype, int storage) {
+  if (B <= 0 || H <= 0 || N <= 0 || head_dim_pad(d) < 0) return 0;
+  return bwd_plan(B, H, N, head_dim_pad(d), dtype, storage).reg ? 0 : dfl_sinkhorn_bias_workspace_size(B, H, N);
+}
+
 int dfl_pending_error(void) {
   if (!g_mailbox_host) return 0;
   const uint32_t w = __atomic_exchange_n(g_mailbox_host, 0u, __ATOMIC_ACQ_REL);
@@ -805,18 +839,10 @@ int dfl_sinkhorn_bwd(const dfl_sinkhorn_bwd_params* p, void* workspace, size_t w
   const size_t need = dfl_sinkhorn_workspace_size(p->B, p->H, p->N);
   if (!workspace || workspace_bytes < need) return fail("workspace too small: need %zu bytes", need);
   if (p->storage < DFL_STORAGE_AUTO || p->storage > DFL_STORAGE_STREAM) return fail("unknown storage %d", p->storage);
-  const int G = group_size(p->B, p->H, p->N);
-  const int elem = p->dtype == DFL_BF16 ? 2 : 4;
-  int CH = ((p->N + 31) / 32) * 32 < 256 ? ((p->N + 31) / 32) * 32 : 256;  // streamed rows per LDS chunk
-  const size_t lds_res = dfl::sinkhorn_bwd_lds_bytes(p->N, DP, elem, G, CH, false);
-  const bool stream_mode = p->storage == DFL_STORAGE_STREAM || (p->storage == DFL_STORAGE_AUTO && lds_res > LDS_LIMIT);
-  size_t lds = lds_res;
-  if (stream_mode) {
-    // the largest chunk (multiple of 32 rows) whose staging fits next to the stripes
-    for (; CH > 32 && dfl::sinkhorn_bwd_lds_bytes(p->N, DP, elem, G, CH, true) > LDS_LIMIT; CH -= 32) {
-    }
-    lds = dfl::sinkhorn_bwd_lds_bytes(p->N, DP, elem, G, CH, true);
-  }
+  const BwdPlan plan = bwd_plan(p->B, p->H, p->N, DP, p->dtype, p->storage);
+  const int G = plan.G, elem = p->dtype == DFL_BF16 ? 2 : 4;
+  const bool stream_mode = plan.stream, reg_mode = plan.reg;
+  const size_t lds = plan.lds;
   if (lds > LDS_LIMIT)
     return fail("N=%d, d=%d, %s storage needs %zu bytes of LDS per workgroup (limit %zu)", p->N, p->d,
                 stream_mode ? "stream" : "resident", lds, LDS_LIMIT);
@@ -853,17 +879,13 @@ int dfl_sinkhorn_bwd(const dfl_sinkhorn_bwd_params* p, void* workspace, size_t w
   if (int rc = refuse_capture(stream, "dfl_sinkhorn_bwd")) return rc;
   if (int rc = acquire_salt(ws, WS_HEADER + xch_words(p->B, p->H, p->N) * 8, stream, &a.salt))
     return hip_fail((hipError_t)rc, "workspace clear launch");
-  a.ch = CH;
-  // the plan in registers where the stripes fit the register tiles (its operands take the stream
-  // region, unused there)
-  const bool reg_mode = !stream_mode && p->storage == DFL_STORAGE_AUTO &&
-                        dfl::sinkhorn_bwd_reg_fits(p->N, DP, G, lds, LDS_LIMIT);
+  a.ch = plan.CH;
   if (p->pos_bins)
     if (int rc = prepare_bins8(p->pos_bins, p->B, p->N, workspace, sinkhorn_bins8_offset(p->B, p->H, p->N),
                                &a.bins8, &a.bins8t, stream))
       return rc;
   // a workspace with room for the bias matrices: the per-element bins lookups and
-  // distances are evaluated once here instead of in every sweep
+  // distances are evaluated once here instead of in every sweep (in registers they are anyway)
   const bool has_bias = (p->pos_bins && p->pos_weight) || (p->x_res && p->w_dist);
   if (!reg_mode && has_bias && workspace_bytes >= need + dfl_sinkhorn_bias_workspace_size(p->B, p->H, p->N)) {
     float* mat = reinterpret_cast<float*>(ws + bias_mat_offset(p->B, p->H, p->N));
@@ -874,7 +896,7 @@ int dfl_sinkhorn_bwd(const dfl_sinkhorn_bwd_params* p, void* workspace, size_t w
     a.bias_matT = matT;
   }
   const bool coop = coop_launch(G, a.B * a.H);
-  if (reg_mode) {
+  if (reg_mode) {  // (its operands take the stream region, unused here)
     const size_t bhn = (size_t)p->B * p->H * np32(p->N);
     unsigned char* at = ws + stream_region_offset(p->B, p->H, p->N, G);
     auto carve = [&](size_t bytes) { unsigned char* q = at; at += bytes; return q; };

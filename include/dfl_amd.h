@@ -163,6 +163,10 @@ int dfl_sinkhorn_fwd(const dfl_sinkhorn_fwd_params* p, void* workspace, size_t w
  * (sinkhorn_kernel.py:1578-1760). */
 size_t dfl_sinkhorn_bias_workspace_size(int B, int H, int N);
 
+/* The part of that extension which dfl_sinkhorn_bwd reads for this shape, head dim, type and
+ * storage: all of it, or 0 where it keeps the plan in registers. */
+size_t dfl_sinkhorn_bwd_bias_workspace_size(int B, int H, int N, int d, int dtype, int storage);
+
 /* Allocation-free variant of dfl_sinkhorn_fwd.  It has no counterpart in the
  * reference: it is for callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).  Same

@@ -205,8 +205,10 @@ def test_backward_bins_outside_table():
     assert_close_rel(got["pos_weight"], np.asarray(want["pos_weight"])[:, :68], 1e-4, "bins-outside:pos_weight")
 
 
+# (d = 32 keeps the plan in registers and reads no matrix; d = 64 does)
+@pytest.mark.parametrize("d", [32, 64])
 @pytest.mark.parametrize("dtype,solver", [(torch.float32, "cg"), (torch.bfloat16, "fixed_point")])
-def test_backward_precomputed_bias_matches_per_element(dtype, solver):
+def test_backward_precomputed_bias_matches_per_element(dtype, solver, d):
     """With the workspace extension (dfl_sinkhorn_bias_workspace_size) the backward
     evaluates the position / geometry bias once and reads it in its sweeps; without it
     every sweep evaluates bins and distances.  Both read the same values, so the
@@ -219,7 +221,7 @@ def test_backward_precomputed_bias_matches_per_element(dtype, solver):
 
     fsa = importlib.import_module("deepfold_amd.flash_sinkhorn_attn")  # the module, not the function
 
-    B, H, N, d = 2, 3, 200, 32
+    B, H, N = 2, 3, 200
     inp = make_inputs(B, H, N, d, seed=91, eps=[0.5, 1.0, 2.0], pos_geo=True)
     g = torch.Generator().manual_seed(92)
     bins = inp["pos_bins"].clone()
@@ -231,16 +233,18 @@ def test_backward_precomputed_bias_matches_per_element(dtype, solver):
     go, gxc = grad_inputs(B, H, N, d, seed=93, with_xc=True)
     go = go * mask[:, :, None]
     kw = dict(ift_solver=solver, ift_iters=12 if solver == "cg" else None)
-    got = {}
+    got, sizes = {}, {}
     saved = fsa._BIAS_WS_MAX
     try:
         for label, cap in (("matrix", saved), ("per_element", -1)):
             fsa._BIAS_WS_MAX = cap
             _lib._ws_cache.clear()  # the next workspace is exactly the requested size
             got[label] = run_gpu_bwd(inp, 6, dtype, go, gxc, mask=mask, **kw)
+            sizes[label] = max(w.numel() for w in _lib._ws_cache.values())
     finally:
         fsa._BIAS_WS_MAX = saved
         _lib._ws_cache.clear()
+    assert (sizes["matrix"] > sizes["per_element"]) == (d == 64)
     for k in got["matrix"]:
         if k in ("pos_weight", "w_dist", "x_res"):
             assert max_rel_err(got["matrix"][k], got["per_element"][k]) <= 1e-6, k
