@@ -54,7 +54,7 @@ template <int DP>
 __global__ void __launch_bounds__(256) balanced_prep_kernel(BalPrepArgs p) {
   const int N = p.N, d = p.d;
   const int Np = ((N + 31) / 32) * 32;
-  sb_clear_steps(p.steps, p.B * p.H, N, p.K);
+  if (p.steps) sb_clear_steps(p.steps, p.B * p.H, N, p.K);
   const size_t e = (size_t)blockIdx.x * 256 + threadIdx.x;
   const size_t row = e / DP;
   const int c = (int)(e % DP);
@@ -496,7 +496,7 @@ __global__ void __launch_bounds__(SB_NT) balanced_scaled_kernel(BalBwdArgs a) {
   if (scaled_bwd<float, true>(a)) balanced_general<32>(fresh_args<BalBwdArgs>());
 }
 
-size_t scaled_step_words(int N) { return sb_step_words(N); }
+size_t scaled_step_words(int N, int DP, int G) { return sb_fits_shape(N, DP, G) ? sb_step_words(N) : 0; }
 
 size_t balanced_bwd_lds_bytes(int N, int DP) {
   (void)DP;

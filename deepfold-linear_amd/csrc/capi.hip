@@ -63,7 +63,7 @@ size_t balanced_bwd_lds_bytes(int N, int DP);
 int balanced_max_tiles(int DP);
 hipError_t launch_balanced_prep(const BalPrepArgs& p, int DP, hipStream_t stream);
 hipError_t launch_balanced_bwd(const BalBwdArgs& a, int DP, size_t lds, size_t limit, hipStream_t stream, bool coop);
-size_t scaled_step_words(int N);
+size_t scaled_step_words(int N, int DP, int G);
 bool sinkhorn_bwd_reg_n(int N, int G);
 bool sinkhorn_bwd_reg_fits(int N, int DP, int G, size_t lds_general, size_t limit);
 hipError_t launch_sinkhorn_bwd_reg(const IftBwdArgs& a, bool bf16_in, size_t lds_general, hipStream_t stream,
@@ -601,7 +601,7 @@ BalWs bal_ws_layout(int B, int H, int N, int d) {
   const size_t op = r256((size_t)B * H * np * DP * 4);
   BalWs w;
   w.steps = WS_HEADER + xch_words(B, H, N) * 8;
-  w.qp = r256(w.steps + (size_t)B * H * dfl::scaled_step_words(N) * 8);
+  w.qp = r256(w.steps + (size_t)B * H * dfl::scaled_step_words(N, DP, G) * 8);
   w.kp = w.qp + op;
   w.qt = w.kp + op;
   w.kt = w.qt + op;
@@ -640,7 +640,7 @@ UnrWs unr_ws_layout(int B, int H, int N, int d) {
   const size_t op = r256((size_t)B * H * np * DP * 4);
   UnrWs w;
   w.steps = WS_HEADER + xch_words(B, H, N) * 8;
-  w.qp = r256(w.steps + (size_t)B * H * dfl::scaled_step_words(N) * 8);
+  w.qp = r256(w.steps + (size_t)B * H * dfl::scaled_step_words(N, DP, G) * 8);
   w.kp = w.qp + op;
   w.qt = w.kp + op;
   w.kt = w.qt + op;
@@ -1228,7 +1228,8 @@ int dfl_balanced_bwd(const dfl_balanced_bwd_params* p, void* workspace, size_t w
   pr.qp = F(L.qp); pr.kp = F(L.kp); pr.qt = F(L.qt); pr.kt = F(L.kt);
   pr.vp = has_h ? F(L.vp) : nullptr; pr.gp = has_h ? F(L.gp) : nullptr; pr.gt = has_h ? F(L.gt) : nullptr;
   pr.dcoef = F(L.dcoef); pr.gxs = F(L.gxs); pr.xs = F(L.xs);
-  pr.steps = reinterpret_cast<uint64_t*>(ws + L.steps); pr.K = p->K_iter;
+  pr.steps = dfl::scaled_step_words(p->N, DP, G) ? reinterpret_cast<uint64_t*>(ws + L.steps) : nullptr;
+  pr.K = p->K_iter;
   hipError_t e = dfl::launch_balanced_prep(pr, DP, (hipStream_t)stream);
   if (e != hipSuccess) return hip_fail(e, "balanced backward prep launch");
   dfl::BalBwdArgs a;
@@ -1240,7 +1241,7 @@ int dfl_balanced_bwd(const dfl_balanced_bwd_params* p, void* workspace, size_t w
   a.dq = p->dq; a.dk = p->dk; a.dv = p->dv; a.dx_part = F(L.dx_part); a.ar_part = F(L.ar_part);
   a.err = err_ref(ws);
   a.xch = reinterpret_cast<uint64_t*>(ws + WS_HEADER);
-  a.steps = reinterpret_cast<uint64_t*>(ws + L.steps);
+  a.steps = pr.steps;
   a.G = G;
   if (int rc = refuse_capture(stream, "dfl_balanced_bwd")) return rc;
   if (int rc = acquire_salt(ws, WS_HEADER + xch_words(p->B, p->H, p->N) * 8, stream, &a.salt))
@@ -1296,7 +1297,8 @@ int dfl_sinkhorn_unrolled_bwd(const dfl_sinkhorn_unrolled_bwd_params* p, void* w
   pr.qp = F(L.qp); pr.kp = F(L.kp); pr.qt = F(L.qt); pr.kt = F(L.kt);
   pr.vp = F(L.vp); pr.gp = F(L.gp); pr.gt = F(L.gt);
   pr.dcoef = F(L.dcoef); pr.gxs = F(L.gxs); pr.xs = F(L.xs); pr.dg = p->dg;
-  pr.steps = reinterpret_cast<uint64_t*>(ws + L.steps); pr.K = p->K_iter;
+  pr.steps = dfl::scaled_step_words(p->N, DP, G) ? reinterpret_cast<uint64_t*>(ws + L.steps) : nullptr;
+  pr.K = p->K_iter;
   hipError_t e = dfl::launch_unrolled_prep(pr, p->dtype == DFL_BF16, DP, (hipStream_t)stream);
   if (e != hipSuccess) return hip_fail(e, "unrolled backward prep launch");
   dfl::UnrBwdArgs a;
@@ -1316,7 +1318,7 @@ int dfl_sinkhorn_unrolled_bwd(const dfl_sinkhorn_unrolled_bwd_params* p, void* w
   a.dx_part = F(L.dx_part); a.dpw_part = F(L.dpw_part); a.dw_part = F(L.dw_part);
   a.err = err_ref(ws);
   a.xch = reinterpret_cast<uint64_t*>(ws + WS_HEADER);
-  a.steps = reinterpret_cast<uint64_t*>(ws + L.steps);
+  a.steps = pr.steps;
   a.G = G;
   if (int rc = refuse_capture(stream, "dfl_sinkhorn_unrolled_bwd")) return rc;
   if (int rc = acquire_salt(ws, WS_HEADER + xch_words(p->B, p->H, p->N) * 8, stream, &a.salt))

@@ -73,8 +73,10 @@ inline size_t ift_lds_bytes(int N, int G) {
   const size_t f = 5 * Np + 3 * loc, m = (loc / 16) * SB_NW * 8 * WAVE;
   return ((Np + 15) / 16) * 16 + (7 * Np + 2 * cpn + 2 * SB_BINS + 2 * (size_t)SB_NW * SK_RT * 16 + (f > m ? f : m)) * 4;
 }
+// The unrolled forms: shapes whose workspace holds the kept words, and calls that run them.
+inline bool sb_fits_shape(int N, int DP, int G) { return DP == 32 && reg_fits(N, G); }
 inline bool sb_fits(int N, int DP, int G, int K, bool bal, size_t limit) {
-  return DP == 32 && K >= 1 && K <= SB_KMAX && reg_fits(N, G) && sb_lds_bytes(N, G, K, bal) + 2048 <= limit;
+  return sb_fits_shape(N, DP, G) && K >= 1 && K <= SB_KMAX && sb_lds_bytes(N, G, K, bal) + 2048 <= limit;
 }
 
 // The kernel's argument struct (its only parameter) for the general sweeps, read anew from where the

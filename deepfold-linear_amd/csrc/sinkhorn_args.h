@@ -148,7 +148,7 @@ struct BalBwdArgs {
   float* dx_part;      // (B,H,N,3) per-head partials
   float* ar_part;      // (B*H*G, 2) per-workgroup d alpha, d r partials
   uint64_t* xch;       // B*H*2*Np exchange words
-  uint64_t* steps;     // sb_step_words(N) per (b,h): the register form's kept exchange words
+  uint64_t* steps;     // sb_step_words(N) per (b,h): the register form's kept exchange words, or null
   ErrRef err;
   int G;
   uint32_t salt;
@@ -192,7 +192,7 @@ struct UnrBwdArgs {
   float* dpw_part;       // (B*H*G, 68)
   float* dw_part;        // (B*H*G)
   uint64_t* xch;
-  uint64_t* steps;       // sb_step_words(N) per (b,h): the register form's kept exchange words
+  uint64_t* steps;       // sb_step_words(N) per (b,h): the register form's kept exchange words, or null
   ErrRef err;
   int G;
   uint32_t salt;
@@ -248,7 +248,7 @@ struct BalPrepArgs {
   float* qp; float* kp; float* qt; float* kt;
   float* vp; float* gp; float* gt;  // null without grad_hc
   float* dcoef; float* gxs; float* xs;
-  uint64_t* steps;     // kept exchange words of the register form, cleared for K iterations
+  uint64_t* steps;     // kept exchange words of the register form, cleared for K iterations (or null)
   int K;
 };
 

@@ -114,6 +114,19 @@ def test_struct_layout_matches_c(lib_path):
             assert getattr(cls, f).offset == c_layout[(sname, f)], (sname, f)
 
 
+def test_kept_words_only_where_the_register_form_runs(lib_path):
+    """The unrolled backward's workspace holds the register form's kept exchange words (12.7 MB at 16
+    heads of 768 tokens) only for shapes that it takes: none at 800 tokens or head dim 64."""
+    from deepfold_amd import _lib
+
+    lib = _lib.load(lib_path)
+    size = lambda n, d: lib.dfl_sinkhorn_unrolled_workspace_size(1, 16, n, d)
+    words = (2 * 64 + 1) * 768 * 8 * 16
+    assert size(768, 32) > size(800, 32) > size(768, 32) - words
+    # the operands of d = 64 are twice those of d = 32: without the words less than twice the size
+    assert size(768, 64) < 2 * (size(768, 32) - words)
+
+
 def test_integration_snippet_matches_binding():
     """The ctypes struct INTEGRATION.md shows a maintainer lists every field of
     dfl_sinkhorn_fwd_params, in order and with the right C types: a struct that
