@@ -963,20 +963,36 @@ __device__ __forceinline__ void flow_sweep(bool online, const T* res, const T* s
 // rank-2 MFMA, four exponentials and four adds a pair: at the headline's 759-token
 // members 1.05-1.35 us a sweep before, about 0.35 us so.  E <= 1, so an entry that
 // underflows is below 2^-126 of its row's largest; while no potential has moved by more than
-// REG_MAX_DRIFT from its base, it stays below 2^-62 of it.  A wave that meets a larger move
-// leaves REG_REDO as its partials; the workgroup then forms its entries anew and repeats the
-// sweep, which nothing has been published of.  Once a row's LSE of the sweep that formed its
-// entries is known, every wave brings them to that common shift (reg_rescale), so the later
-// partials of the waves are plain sums.
-constexpr float REG_MAX_DRIFT = 32.f;  // log2 units
+// REG_MAX_DRIFT from its base, it stays below 2^-38 of it (of 768 such, 2^-28).  A wave that meets a larger move
+// leaves REG_REDO as its partials, and the half-iteration, which nothing has been published of,
+// is repeated: with all bases and shifts moved by a constant, which changes no entry, where the
+// moves lie within the bound of one (small eps moves every potential alike), else with the
+// entries formed anew.  Once a row's LSE of the sweep that formed its entries is known, every wave
+// brings them to that common shift (reg_rescale), so the later partials of the waves are plain sums.
+constexpr float REG_MAX_DRIFT = 44.f;  // log2 units, as all of these
+constexpr float REG_SLACK = 10.f;      // least that a common move leaves of the bound
+constexpr float REG_MAX_MOVE = 64.f;   // largest common move: the entries keep the rounding of the
+                                       // exponents that they were formed with
+// Forming costs 5 us (256 tokens) to 24 us (768, bins and geometry), a repeated half-iteration 2.2 us.
+// Starting potentials further than REG_FAR from kappa log nu, or an eps below REG_SHARP_EPS (unit-variance
+// queries and keys then spread the first update by 40 and more), would have the entries formed in
+// vain: the first iteration runs on the logits instead, 0.7 us a half more than in scaling form.
+// Forward us with rank-2 sweeps on the logits throughout / with every move beyond 32 formed anew / so, bf16,
+// eps 0.5, three log nu at -70: 16 heads of 389, K 7, bins and geometry 57 / 68 / 57; 16 heads of 768,
+// K 20, bins and geometry 162 / 165 / 142; eps 0.1 57 / 68 / 58 and 161 / 167 / 144; eps 0.05 57 / 68 / 59
+// and 161 / 191 / 154; eps 0.02 57 / 80 / 64 and 162 / 264 / 185 (there the spread keeps moving);
+// warm start of 20 nats 58 / 80 / 60 and 162 / 189 / 145.
+constexpr float REG_FAR = 24.f;
+constexpr float REG_SHARP_EPS = 0.075f;
 constexpr float REG_REDO = 3.0e38f;
 __device__ __forceinline__ bool reg_redo(float sum) { return sum >= 2.9e38f; }
 
 // X holds the logits S (log2; anything in slots of tiles the wave does not have): turns them
-// into E with the potentials pot (by streamed index) as base and the wave's row maxima as shift,
+// into E with the potentials pot (by streamed index) as base and the wave's row maxima as shift
+// (KEEP: leaves the logits),
 // and leaves the rows' partials p_w = sh + log2 sum_(its j) E_qj (NEG_BIG for an empty sum) as in
 // flow_chunk.  The potentials enter by one rank-2 MFMA per pair.
-template <int KS, int NRM, int NW>
+template <int KS, int NRM, int NW, bool KEEP>
 __device__ __forceinline__ void reg_online(f32x4 (&X)[NRM * KS], float (&sh)[NRM], int nr, int n_tiles,
                                            const float* pot, float* part) {
   const int lane = threadIdx.x & (WAVE - 1);
@@ -1012,7 +1028,7 @@ __device__ __forceinline__ void reg_online(f32x4 (&X)[NRM * KS], float (&sh)[NRM
 #pragma unroll
         for (int q = 0; q < 4; ++q) x[q] = fast_exp2(x[q]);
         ss += (x[0] + x[1]) + (x[2] + x[3]);
-        X[r * KS + k] = x;
+        if constexpr (!KEEP) X[r * KS + k] = x;
       }
       ss = sum_groups(ss);
       // (a NaN passes on; an empty sum is NEG_BIG)

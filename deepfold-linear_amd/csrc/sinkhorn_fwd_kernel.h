@@ -295,7 +295,7 @@ __global__ void __launch_bounds__(FWD_NT) sinkhorn_fwd_kernel(SinkFwdArgs a) {
   constexpr bool HIST = BAL || MODE == FWD_UOT_HIST || MODE == FWD_HIST_REG;
   constexpr bool REG = !STREAM && (MODE == FWD_UOT_REG || MODE == FWD_HIST_REG || MODE == FWD_BAL_REG);
   extern __shared__ __align__(16) unsigned char smem[];
-  __shared__ int s_flag, s_tmp, s_local;
+  __shared__ int s_flag, s_tmp, s_local, s_far;
   __shared__ unsigned s_du, s_dv;
   __shared__ int s_cnt;
   __shared__ int s_flagp[2];  // resident dataflow: expired waits of the half-iterations, by parity
@@ -307,7 +307,7 @@ __global__ void __launch_bounds__(FWD_NT) sinkhorn_fwd_kernel(SinkFwdArgs a) {
   const int Np = ((N + 31) / 32) * 32;
   constexpr bool bal = BAL;
   const bool has_v = !BAL || (a.v != nullptr && a.o_avg != nullptr);  // UOT mode always has V
-  if (threadIdx.x == 0) { s_flag = 0; s_du = 0u; s_dv = 0u; s_cnt = 0; s_local = 1; s_flagp[0] = s_flagp[1] = 0; }
+  if (threadIdx.x == 0) { s_flag = 0; s_du = 0u; s_dv = 0u; s_cnt = 0; s_local = 1; s_far = 0; s_flagp[0] = s_flagp[1] = 0; }
   if (blockIdx.x == 0 && threadIdx.x == 0)
     __hip_atomic_store(a.err.ws + 1, a.salt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 
@@ -371,6 +371,13 @@ __global__ void __launch_bounds__(FWD_NT) sinkhorn_fwd_kernel(SinkFwdArgs a) {
   const T* Qp = STREAM ? reinterpret_cast<const T*>(a.qp) + bh * Np * DP : nullptr;
   const T* Kp = STREAM ? reinterpret_cast<const T*>(a.kp) + bh * Np * DP : nullptr;
   const int r_lo = t0 * 16;
+  // register storage (at most 768 tokens): log nu of all columns, in flight with Q and K
+  float lnu_i[2] = {0.f, 0.f};
+  if constexpr (REG && !BAL) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+      if ((int)threadIdx.x + k * FWD_NT < n) lnu_i[k] = a.log_nu[bh * N + threadIdx.x + k * FWD_NT];
+  }
   if constexpr (STREAM) {
     stage_rows<T, DP>(QS, Qp + (size_t)r_lo * DP, DP, nr * 16, DP, loc);
     stage_rows<T, DP>(KS, Kp + (size_t)r_lo * DP, DP, nr * 16, DP, loc);
@@ -410,6 +417,16 @@ __global__ void __launch_bounds__(FWD_NT) sinkhorn_fwd_kernel(SinkFwdArgs a) {
   }
   if constexpr (REG)
     for (int i = threadIdx.x; i < 2 * cpn; i += FWD_NT) mulU[i] = 0.f;  // both arrays
+  // the column potentials' first move, but for their column's LSE, which the cost decides
+  if constexpr (REG && !BAL) {
+    bool far_move = eps < REG_SHARP_EPS;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const int i = threadIdx.x + k * FWD_NT;  // (vecV[i] is this thread's)
+      far_move = far_move || (i < n && valid[i] && !(fabsf(kappa * LOG2E * lnu_i[k] - vecV[i]) <= REG_FAR));
+    }
+    if (far_move && a.K_iter >= 2) s_far = 1;
+  }
   const float w_h = bal ? w_bal : (a.w_dist ? a.w_dist[h] : 0.f);
   const bool use_geo = GEN && (a.x != nullptr) && (w_h != 0.f);
   const bool use_pos = GEN && (a.bins8 != nullptr) && (a.pos_w != nullptr);
@@ -667,11 +684,11 @@ __global__ void __launch_bounds__(FWD_NT) sinkhorn_fwd_kernel(SinkFwdArgs a) {
       // v_j = kappa (log nu_j - LSE_i(L_ij + u_i)) for my columns.  ONLINE: X holds logits, to be
       // turned into entries with the present potentials as base, else entries at the rows' common
       // shifts.  fin: the UOT mode's last row sweep (exact log Z and row maxima), which publishes
-      // nothing.  Returns 0, 1 if the entries have to be formed anew for it (nothing is published
-      // then), or -1 on an expired wait.
+      // nothing.  Returns 0, 1 if potentials have moved too far from their bases for it (nothing is
+      // published then), or -1 on an expired wait.
       auto half = [&](auto rowc, auto onl, f32x4(&X)[NRM * KSL], float(&sh)[NRM], float(&base)[NB], float& shift, int it,
                       bool fin) __attribute__((always_inline)) -> int {
-        constexpr bool ONLINE = decltype(onl)::value;
+        constexpr bool ONLINE = decltype(onl)::value != 0, KEEP = decltype(onl)::value == 2;
         constexpr bool ROW = decltype(rowc)::value;
         ++phase;
         const uint32_t tag = salt | phase;
@@ -696,7 +713,7 @@ __global__ void __launch_bounds__(FWD_NT) sinkhorn_fwd_kernel(SinkFwdArgs a) {
               mul[i] = valid[i] ? 1.f : 0.f;
             }
           }
-          reg_online<KSL, NRM, FWD_NW>(X, sh, nr, n_tiles, pot, part);
+          reg_online<KSL, NRM, FWD_NW, KEEP>(X, sh, nr, n_tiles, pot, part);
         } else if (redo) {
           if (lane < 16)
             for (int r = 0; r < nr; ++r) part[(r * 16 + lane) * FWD_NW + wave] = REG_REDO;
@@ -748,8 +765,9 @@ __global__ void __launch_bounds__(FWD_NT) sinkhorn_fwd_kernel(SinkFwdArgs a) {
       int it = 0;
       float shiftR = 0.f, shiftC = 0.f;  // common shifts of local row / column qc
       bool row_turn = !BAL, done = false;
-      const std::integral_constant<bool, true> online_c{};
-      const std::integral_constant<bool, false> scaled_c{};
+      const std::integral_constant<int, 0> scaled_c{};
+      const std::integral_constant<int, 1> online_c{};
+      const std::integral_constant<int, 2> logits_c{};
       // to the next half-iteration; true after the last one
       auto advance = [&]() __attribute__((always_inline)) -> bool {
         if (!BAL && it == a.K_iter) return true;  // the final row sweep
@@ -757,18 +775,67 @@ __global__ void __launch_bounds__(FWD_NT) sinkhorn_fwd_kernel(SinkFwdArgs a) {
         row_turn = !row_turn;
         return it == a.K_iter && (BAL || !reg_tail);
       };
-      while (true) {
-        form();
-        int st = 0;
-        for (int z = 0; z < 2 && !done; ++z) {
-          st = row_turn ? half(row_c, online_c, XR, shR, baseV, shiftR, it, !BAL && it == a.K_iter)
-                        : half(col_c, online_c, XC, shC, baseU, shiftC, it, false);
-          if (st < 0) return false;
-          done = advance();
+      // After a half-iteration that returned 1: moves all bases and shifts of its orientation by a
+      // constant that leaves the moves well within the bound, if one does.
+      auto rebase = [&]() __attribute__((always_inline)) -> bool {
+        const float* pot = row_turn ? vecV : vecU;
+        float lo = 3.0e38f, hi = -3.0e38f;
+#pragma unroll
+        for (int s = 0; s < NB; ++s) {
+          const int e = s * WAVE + lane, i = (wave + FWD_NW * (e >> 4)) * 16 + (e & 15);
+          if (e < 16 * KSL && i < n && valid[i]) {
+            const float m = pot[i] - (row_turn ? baseV[s] : baseU[s]);
+            const bool fine = fabsf(m) < 1.0e6f;  // (a NaN, an infinity or NEG_BIG has no common move)
+            lo = fminf(lo, fine ? m : -3.0e38f);
+            hi = fmaxf(hi, fine ? m : 3.0e38f);
+          }
         }
-        if (done) break;
-        reg_rescale<KSL, NRM>(XR, shR, nr, lse_r);
-        reg_rescale<KSL, NRM>(XC, shC, nr, lse_c);
+#pragma unroll
+        for (int o = 1; o < WAVE; o <<= 1) {
+          lo = fminf(lo, __shfl_xor(lo, o, WAVE));
+          hi = fmaxf(hi, __shfl_xor(hi, o, WAVE));
+        }
+        if (lane == 0) { scratch[wave] = lo; scratch[FWD_NW + wave] = hi; }  // (both slots' partials are read)
+        __syncthreads();
+#pragma unroll
+        for (int w_ = 0; w_ < FWD_NW; ++w_) {
+          lo = fminf(lo, scratch[w_]);
+          hi = fmaxf(hi, scratch[FWD_NW + w_]);
+        }
+        const float by = rintf(0.5f * lo + 0.5f * hi);
+        if (!(0.5f * hi - 0.5f * lo <= REG_MAX_DRIFT - REG_SLACK && fabsf(by) <= REG_MAX_MOVE)) return false;
+        const float byR = row_turn ? by : 0.f, byC = row_turn ? 0.f : by;
+#pragma unroll
+        for (int s = 0; s < NB; ++s) { baseV[s] += byR; baseU[s] += byC; }
+#pragma unroll
+        for (int r = 0; r < NRM; ++r) { shR[r] += byR; shC[r] += byC; }
+        shiftR += byR;
+        shiftC += byC;
+        return true;
+      };
+      bool fresh = true;  // the entries have to be formed
+      while (true) {
+        int st = 0;
+        if (fresh) {
+          form();
+          if constexpr (!BAL)
+            if (s_far) {  // the first iteration runs on the logits
+              if (half(row_c, logits_c, XR, shR, baseV, shiftR, it, false) < 0) return false;
+              advance();
+              if (half(col_c, logits_c, XC, shC, baseU, shiftC, it, false) < 0) return false;
+              advance();
+              if (threadIdx.x == 0) s_far = 0;  // (read by every wave two barriers ago; next after a barrier)
+            }
+          for (int z = 0; z < 2 && !done; ++z) {
+            st = row_turn ? half(row_c, online_c, XR, shR, baseV, shiftR, it, !BAL && it == a.K_iter)
+                          : half(col_c, online_c, XC, shC, baseU, shiftC, it, false);
+            if (st < 0) return false;
+            done = advance();
+          }
+          if (done) break;
+          reg_rescale<KSL, NRM>(XR, shR, nr, lse_r);
+          reg_rescale<KSL, NRM>(XC, shC, nr, lse_c);
+        }
         while (true) {
           st = row_turn ? half(row_c, scaled_c, XR, shR, baseV, shiftR, it, !BAL && it == a.K_iter)
                         : half(col_c, scaled_c, XC, shC, baseU, shiftC, it, false);
@@ -777,10 +844,11 @@ __global__ void __launch_bounds__(FWD_NT) sinkhorn_fwd_kernel(SinkFwdArgs a) {
         }
         if (st < 0) return false;
         if (done) break;
-        // the entries are formed anew and the half-iteration repeated
+        // the half-iteration is repeated
         __syncthreads();
         if (threadIdx.x == 0) s_flagp[phase & 1] = 0;
         --phase;
+        fresh = !rebase();
         __syncthreads();
       }
       if (!reg_tail) return true;
