@@ -230,3 +230,20 @@ def test_pipeline_tile_edges(B, H, N, d, K, lengths):
     # a single row's plan is 1 whatever the cost: its cost and marginal gradients vanish
     names = ("V", "G", "x") if N == 1 else ("C", "mu", "nu", "V", "G", "x")
     _cmp(_grads(fn, {"C": C, "mu": lmu, "nu": lnu, "V": V, "G": G, "x": x}), names)
+
+
+@pytest.mark.parametrize("N", [70, 512, 1100])
+def test_transport_plan_rounding(N):
+    """T_norm does not depend on u, so neither does its rounding.  2-norm bound: the exponent
+    C log2 e / eps + v log2 e, both rounded at magnitudes below 16 (half an ulp 4.8e-7, rms 2.8e-7 each), times
+    ln 2, is 2.7e-7 of an entry; its exponential and two products add 0.6e-7: 2.8e-7 in all, 3.3e-7 asked."""
+    from deepfold_amd import compute_transport_output
+
+    C, _, lnu, eps, g = _case(1, 4, N, seed=N)
+    V, G = (torch.randn(1, 4, N, 16, generator=g) for _ in range(2))
+    lu, lv = -40.0 + torch.randn(1, 4, N, generator=g), lnu
+    t = lambda x: x.to(DEV)
+    _, T, _ = compute_transport_output(t(V), t(G), t(lu), t(lv), t(C), t(eps))
+    _, want, _ = dref.compute_transport_output(V.double(), G.double(), lu.double(), lv.double(), C.double(), eps.double())
+    err = float((T.cpu().double() - want).norm() / want.norm())
+    assert err <= 3.3e-7, err
