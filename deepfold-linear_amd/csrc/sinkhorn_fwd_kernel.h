@@ -680,6 +680,7 @@ __global__ void __launch_bounds__(FWD_NT) sinkhorn_fwd_kernel(SinkFwdArgs a) {
         block(std::integral_constant<bool, true>{}, XR);
         block(std::integral_constant<bool, false>{}, XC);
       };
+      float sumR = -1.f;  // sum of local row qc in the last row sweep, -1 if that formed the entries
       // One half-iteration.  ROW: u_i = kappa (log mu_i - LSE_j(L_ij + v_j)) for my rows, else
       // v_j = kappa (log nu_j - LSE_i(L_ij + u_i)) for my columns.  ONLINE: X holds logits, to be
       // turned into entries with the present potentials as base, else entries at the rows' common
@@ -735,7 +736,9 @@ __global__ void __launch_bounds__(FWD_NT) sinkhorn_fwd_kernel(SinkFwdArgs a) {
             const float ss = reg_sum<FWD_NW>(part, qc);
             pub = !reg_redo(ss);
             l2 = ss <= 0.f ? NEG_BIG : shift + fast_log2(ss);
+            if constexpr (ROW) sumR = ss;
           }
+          if constexpr (ONLINE && ROW) sumR = -1.f;
           if (!pub) {
             atomicOr(&s_flagp[phase & 1], 2);
           } else {
@@ -852,12 +855,15 @@ __global__ void __launch_bounds__(FWD_NT) sinkhorn_fwd_kernel(SinkFwdArgs a) {
         __syncthreads();
       }
       if (!reg_tail) return true;
-      // ---- Tail: P_ij = E_ij w_j exp2(sh_i - lse_i) with the row LSE of the last row sweep;
+      // ---- Tail: P_ij = E_ij w_j / sum_j E_ij w_j with the sum of the last row sweep, or exp2(sh_i - lse_i)
+      // where that formed the entries.  The sum, and not its logarithm, whose rounding is 2e-7 of an entry:
+      // x_centroid of 2x8 heads of 768 tokens 3.6e-7 from float64 with the logarithm, 2.6e-7 so;
       // each wave sums its streamed tiles, the partials meet in LDS and the wave r writes
       // resident tile r.  No logit or bias is recomputed.
       if constexpr (DP == 32) {
         T* VT = QS;  // [DP][Np]: every wave has passed its last sweep
         if (has_v) stage_rows_t<T, DP>(VT, Vg, a.sn, n, d, Np);
+        if (qc < nr * 16) lmu_l[qc] = sumR < 0.f ? -1.f : 1.f / sumR;
         if (!BAL && qc < nr * 16) {
           float mm = NEG_BIG;
 #pragma unroll
@@ -876,7 +882,8 @@ __global__ void __launch_bounds__(FWD_NT) sinkhorn_fwd_kernel(SinkFwdArgs a) {
 #pragma unroll
         for (int r = 0; r < NRM; ++r) {
           if (r < nr) {
-            const float cr = fast_exp2(shR[r] - lse_r[r * 16 + (lane & 15)]);
+            const float inv = lmu_l[r * 16 + (lane & 15)];
+            const float cr = inv >= 0.f ? inv : fast_exp2(shR[r] - lse_r[r * 16 + (lane & 15)]);
 #pragma unroll
             for (int k = 0; k < KSL; ++k) {
               const int st = wave + FWD_NW * k;
