@@ -1,11 +1,11 @@
 // Flash-Sinkhorn IFT backward with the plan in registers (scaled_bwd.h): a translation unit of its
-// own so that it compiles in parallel with the general one, which serves a group out of range.
+// own so that it compiles in parallel with the general one, whose sweeps serve a group out of range.
 //
 // Bound by the latency of the solve's exchanges (two per iteration, about 2 us each with the sweep
 // between them) and by the two passes of the cost gradient.  One multiply-add per element and sweep
 // in place of a matrix product, a bias and an exponential: 16 heads of 389 tokens with bins and
-// geometry, 7 fixed-point iterations: 229 us and 15 us for the bias matrix -> 101 us (no bias
-// matrix); 16 heads of 768 tokens, 20 iterations: 180 -> 155 us.
+// geometry, 7 fixed-point iterations: 229 us and 15 us for the bias matrix -> 85 us (no bias
+// matrix); 2x8 heads of 768 tokens, 20 CG iterations: 180 -> 149 us.
 #include "scaled_bwd.h"
 
 namespace dfl {

@@ -148,7 +148,9 @@ def test_register_balanced(B, H, N, d, K, eps, lengths):
     (1, 4, 40, 16, 64, 1.0, None, 1e-4),          # the most iterations whose vectors are kept
     (1, 4, 40, 16, 65, 1.0, None, 1e-4),          # one more: the general sweeps
     (2, 8, 300, 32, 1, 0.5, [300, 163], 1e-4),    # a single iteration: no recurrence
-    (1, 8, 130, 32, 3, 0.03, [117], 1e-3),        # factors out of range: the general sweeps as a call
+    (1, 8, 130, 32, 3, 0.03, [117], 1e-3),        # sharp plans, inside the factors' range
+    (1, 8, 130, 32, 3, 0.003, [117], 1e-3),       # factors out of range: the general sweeps
+    (1, 16, 256, 32, 20, 0.003, None, 1e-3),
 ])
 def test_register_balanced_gradients(B, H, N, d, K, eps, lengths, tol):
     from deepfold_amd import balanced_sinkhorn_transport_dual
@@ -165,6 +167,12 @@ def test_register_balanced_gradients(B, H, N, d, K, eps, lengths, tol):
         for b, n in enumerate(lengths):
             mask[b, :n] = 1
     wx, wh = torch.randn(B, H, N, 3, generator=g), torch.randn(B, H, N, d, generator=g)
+    if eps < 0.03:  # u of the last iteration against the initial zero: a row factor
+        n = lengths[0] if lengths else N
+        f = lambda t: t[:, :, :n].double()
+        u = bt.sinkhorn_cpu(f(leaves["Q"]), f(leaves["K"]), leaves["x"][:, :n].double(), e.double(), leaves["al"].double(),
+                            leaves["r"].double(), None, n, K, return_plan=True)[2]
+        assert float(u.abs().amax(-1).min()) > MAX_FACTOR  # every head
     grads = []
     for fn, conv in ((bt.balanced_transport_dual, lambda t: None if t is None else t.double()),
                      (balanced_sinkhorn_transport_dual, lambda t: None if t is None else t.to(DEV))):
@@ -216,7 +224,7 @@ def test_register_unrolled_gradients(B, H, N, d, K, lengths):
     (1, 2, 17, 32, 0.0, True, None, torch.float32, 1e-4),          # members without a tile
     (2, 8, 300, 24, 0.0, False, [300, 161], torch.float32, 1e-4),  # three tiles a member; padded columns
     (1, 4, 150, 32, 0.0, True, None, torch.bfloat16, 2e-2),
-    (1, 4, 90, 32, 60.0, True, None, torch.float32, 1e-3),         # row sums out of range: the general sweeps as a call
+    (1, 4, 90, 32, 60.0, True, None, torch.float32, 1e-3),         # row sums out of range: the general sweeps
 ])
 def test_register_ift_gradients(B, H, N, d, v_scale, geo, lengths, dtype, tol, solver, iters, mode):
     from test_gpu_sinkhorn_bwd import compare, grad_inputs, run_gpu_bwd
